@@ -15,7 +15,7 @@
 // The top-E keeps a row of up to 16384 distances in the registers of 1024
 // threads and finds the E-th smallest by a 4-pass radix select over the
 // distances' order-preserving 32-bit keys (LDS histograms), then sorts only
-// the E survivors; longer rows use the chunked bitonic kernel.
+// the E survivors; longer rows are streamed once against a running threshold.
 #include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -29,8 +29,7 @@ namespace swann {
 namespace {
 
 constexpr int kTM = 64, kTN = 64, kTK = 16;   // GEMM tile
-constexpr int kTopBuf = 4096;                 // pairs held in LDS by the top-E kernel
-constexpr int kTopBlock = 256;
+constexpr int kTopBuf = 4096;                 // twice the largest E
 constexpr int kRadBlock = 1024, kRadPer = 16; // radix top-E: rows of up to 16384
 constexpr int kRadMaxE = 2048;
 constexpr int kMaxSplit = 16;
@@ -274,6 +273,27 @@ __global__ __launch_bounds__(256) void split_finish(const float* __restrict__ pa
     Dm[i] = metric == SWANN_METRIC_IP ? 1.0f - s : (bn[nn] - 2.0f * s) + an[m];
 }
 
+// A wave's 64 (d, id) pairs in ascending order, in registers: a bitonic network
+// over the lanes (padding entries sort last), no barriers.
+__device__ __forceinline__ void wave_sort(float& d, int& id) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int size = 2; size <= 64; size <<= 1) {
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            const float d2 = __shfl_xor(d, stride, 64);
+            const int id2 = __shfl_xor(id, stride, 64);
+            // both lanes of a pair decide the same swap, from the lower
+            // lane's element (so a pair the order cannot rank, NaN against
+            // NaN, is swapped or kept whole, never duplicated)
+            const bool up = (lane & size) == 0;
+            const bool sw = (lane & stride) == 0 ? up != lt(d, id, d2, id2)
+                                                 : up != lt(d2, id2, d, id);
+            if (sw) { d = d2; id = id2; }
+        }
+    }
+}
+
 // Row top-E for rows of N <= kRadBlock*kRadPer: radix select of the E-th key,
 // then a bitonic sort of the E survivors by (d, index).
 __global__ __launch_bounds__(kRadBlock) void row_topk_radix(const float* __restrict__ Dm,
@@ -394,27 +414,12 @@ __global__ __launch_bounds__(kRadBlock) void row_topk_radix(const float* __restr
     }
     // ---- sort the E survivors by (d, index) ----
     if (E <= 64) {
-        // one wave, in registers: a bitonic network over 64 lanes (lanes
-        // past E hold the padding entry and sort last), no barriers
+        // one wave, in registers (lanes past E hold the padding entry)
         __syncthreads();
         if (wave != 0) return;
         float d = lane < E ? sd[lane] : pad_d();
         int id = lane < E ? si[lane] : INT32_MAX;
-#pragma unroll
-        for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                const float d2 = __shfl_xor(d, stride, 64);
-                const int id2 = __shfl_xor(id, stride, 64);
-                // both lanes of a pair decide the same swap, from the lower
-                // lane's element (so a pair the order cannot rank, NaN
-                // against NaN, is swapped or kept whole, never duplicated)
-                const bool up = (lane & size) == 0;
-                const bool sw = (lane & stride) == 0 ? up != lt(d, id, d2, id2)
-                                                     : up != lt(d2, id2, d, id);
-                if (sw) { d = d2; id = id2; }
-            }
-        }
+        wave_sort(d, id);
         if (lane < E) {
             oi[r * E + lane] = id;
             if (od) od[r * E + lane] = d;
@@ -446,56 +451,304 @@ __global__ __launch_bounds__(kRadBlock) void row_topk_radix(const float* __restr
     }
 }
 
-// Bitonic sort of kTopBuf (d, i) pairs in LDS, ascending.
-__device__ void lds_sort(float* sd, int* si, int n) {
-    for (int size = 2; size <= n; size <<= 1) {
+// Row top-E for longer rows (an entry pool or a whole corpus): one pass over
+// the row against a running threshold.  A workgroup streams its share of the
+// row 2,048 distances at a time, the next two groups' loads in flight, appends
+// those that rank below the E-th best so far to a buffer in LDS, and cuts the
+// buffer back to its E best when another group might not fit (stream_cut: radix
+// select, exact, ties to the lower index).  After the first cut only about
+// E ln(N / 2048) of a row's N distances are appended, so the pass is bound by
+// reading the matrix; 33 KB of LDS is four workgroups a CU, 64 KB of loads in
+// flight on each.  (Sorting the row 4,096 at a time instead: 2,000 rows of
+// 131,072, E = 32, took 17.2 ms; this takes 0.30 ms, 3.5 TB/s of the matrix;
+// 1,024 rows of 400,003, E = 10: 26.8 against 0.35 ms, 4.6 TB/s.)
+constexpr int kStBlock = 256, kStPer = 8, kStGroup = kStBlock * kStPer;
+constexpr int kStBuf = 2 * kStGroup;
+constexpr int kStOwn = kStBuf / kStBlock;      // buffer entries a thread holds in a cut
+static_assert(kTopBuf / 2 + kStGroup <= kStBuf, "after a cut a group fits");
+
+struct StreamLds {
+    float d[kStBuf];
+    int i[kStBuf];
+    unsigned hist[256];
+    unsigned bucket, before, tie;
+    int cnt, wcnt[2][kStBlock / 64];
+};
+
+// One radix select over the workgroup's values u(j), j < kStOwn a thread, those
+// with in(j): the value of rank `need` (from 1), and how many rank before it.
+template <class U, class In>
+__device__ __forceinline__ void stream_rank(StreamLds& L, U u, In in, int need, unsigned* value,
+                                            int* less) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    unsigned prefix = 0u, pmask = 0u;
+    const int need0 = need;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+        L.hist[tid] = 0u;
+        __syncthreads();
+        // values that share their leading bits fall into a few bins: a wave's
+        // lanes of its first two bins add with one atomic each
+#pragma unroll
+        for (int j = 0; j < kStOwn; ++j) {
+            const unsigned bin = (u(j) >> shift) & 255u;
+            bool pend = in(j) && (u(j) & pmask) == prefix;
+#pragma unroll
+            for (int peel = 0; peel < 2; ++peel) {
+                const uint64_t act = __ballot(pend);
+                if (act == 0) break;
+                const unsigned b0 = __builtin_amdgcn_readlane(bin, __builtin_ctzll(act));
+                const uint64_t same = __ballot(pend && bin == b0);
+                if (pend && bin == b0) {
+                    if (lane == __builtin_ctzll(same))
+                        atomicAdd(&L.hist[b0], (unsigned)__builtin_popcountll(same));
+                    pend = false;
+                }
+            }
+            if (pend) atomicAdd(&L.hist[bin], 1u);
+        }
+        __syncthreads();
+        if (tid < 64) {
+            unsigned h[4], run = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { h[j] = L.hist[lane * 4 + j]; run += h[j]; }
+            unsigned incl = run;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned o = __shfl_up(incl, off, 64);
+                if (lane >= off) incl += o;
+            }
+            unsigned before = incl - run;
+            if (before < (unsigned)need && incl >= (unsigned)need) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (before + h[j] >= (unsigned)need) {
+                        L.bucket = lane * 4 + j;
+                        L.before = before;
+                        break;
+                    }
+                    before += h[j];
+                }
+            }
+        }
+        __syncthreads();
+        prefix |= L.bucket << shift;
+        pmask |= 0xFFu << shift;
+        need -= (int)L.before;
+    }
+    *value = prefix;
+    *less = need0 - need;
+}
+
+// Cut the buffer's `n` entries (n >= E) to the E best in (distance, index)
+// order, in place and unsorted; returns the E-th best's key.  Ends with a
+// barrier and L.cnt == E.
+__device__ __forceinline__ unsigned stream_cut(StreamLds& L, int n, int E) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    float d[kStOwn];
+    int id[kStOwn];
+#pragma unroll
+    for (int j = 0; j < kStOwn; ++j) {
+        const int i = tid + j * kStBlock;
+        d[j] = i < n ? L.d[i] : 0.f;
+        id[j] = i < n ? L.i[i] : 0;
+    }
+    auto in = [&](int j) { return tid + j * kStBlock < n; };
+    auto key = [&](int j) { return dkey(d[j]); };
+    unsigned T;
+    int less;
+    stream_rank(L, key, in, E, &T, &less);
+    // copies of T: the E - less lowest indices stay
+    auto eq = [&](int j) { return in(j) && key(j) == T; };
+    if (tid == 0) { L.tie = 0u; L.cnt = 0; }
+    __syncthreads();
+    int neq = 0;
+#pragma unroll
+    for (int j = 0; j < kStOwn; ++j) neq += __builtin_popcountll(__ballot(eq(j)));
+    if (lane == 0 && neq) atomicAdd(&L.tie, (unsigned)neq);
+    __syncthreads();
+    unsigned last = 0xFFFFFFFFu;
+    if ((int)L.tie > E - less) {                // uniform
+        int unused;
+        stream_rank(L, [&](int j) { return (unsigned)id[j]; }, eq, E - less, &last, &unused);
+    }
+#pragma unroll
+    for (int j = 0; j < kStOwn; ++j) {
+        const bool keep = in(j) && (key(j) < T || (key(j) == T && (unsigned)id[j] <= last));
+        const uint64_t m = __ballot(keep);
+        if (m == 0) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&L.cnt, __builtin_popcountll(m));
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (keep) {
+            const int at = base + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+            L.d[at] = d[j];
+            L.i[at] = id[j];
+        }
+    }
+    __syncthreads();
+    return T;
+}
+
+// Workgroup (row, part): the E best of columns [N part / parts, N (part + 1) /
+// parts) of the row.  One part writes the sorted result.  With more, each
+// leaves its E best, unsorted, at the start of the columns it has read (E
+// distances, then E indices; a part has at least 4 E columns), and row_topk_join
+// takes those (JOIN).
+template <bool JOIN>
+__device__ __forceinline__ void row_topk_body(float* __restrict__ row, int64_t N, int E, int parts,
+                                              int part, int32_t* __restrict__ oi,
+                                              float* __restrict__ od) {
+    __shared__ StreamLds L;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t c0 = JOIN ? 0 : N * part / parts;
+    const int64_t c1 = JOIN ? (int64_t)parts * E : N * (part + 1) / parts;
+    const int64_t len = c1 - c0;
+    auto load = [&](int64_t g, float* v, int* id) {
+#pragma unroll
+        for (int j = 0; j < kStPer; ++j) {
+            const int64_t c = g + tid + j * kStBlock;
+            const bool ok = c < len;
+            if constexpr (JOIN) {
+                const int64_t p = ok ? c / E : 0, k = ok ? c - p * E : 0;
+                const float* at = row + N * p / parts;
+                v[j] = at[k];
+                id[j] = reinterpret_cast<const int*>(at + E)[k];
+            } else {
+                v[j] = row[c0 + (ok ? c : 0)];
+            }
+        }
+    };
+    const int wave = tid >> 6;
+    unsigned T = 0u;
+    bool full = false;                          // T holds: E entries rank at or below it
+    int have = 0;                               // entries in the buffer (uniform)
+    const int limit = E + 512 < kStGroup ? (E + 512 > 1024 ? E + 512 : 1024) : kStGroup;
+    float v[kStPer], v1[kStPer], v2[kStPer];
+    int id[kStPer], i1[kStPer], i2[kStPer];
+    load(0, v1, i1);
+    load(kStGroup, v2, i2);
+    int par = 0;
+    for (int64_t g = 0; g < len || have > E; g += kStGroup) {
+        if (have > limit || g >= len) {         // (the last cut: the row is read)
+            __syncthreads();                    // the last group's entries are written
+            T = stream_cut(L, have, E);
+            full = true;
+            have = E;
+            if (g >= len) break;
+        }
+#pragma unroll
+        for (int j = 0; j < kStPer; ++j) {
+            v[j] = v1[j]; v1[j] = v2[j];
+            if constexpr (JOIN) { id[j] = i1[j]; i1[j] = i2[j]; }
+            else id[j] = (int)(c0 + g) + tid + j * kStBlock;
+        }
+        load(g + 2 * kStGroup, v2, i2);
+        // an entry that ties the E-th best comes after it in the row and
+        // ranks after it; joining parts, their entries are in no order, and
+        // the cut decides
+        unsigned on = 0u;
+        int w = 0;
+#pragma unroll
+        for (int j = 0; j < kStPer; ++j) {
+            const unsigned k = dkey(v[j]);
+            const bool p = g + tid + j * kStBlock < len && (!full || (JOIN ? k <= T : k < T));
+            on |= (p ? 1u : 0u) << j;
+            w += __builtin_popcountll(__ballot(p));
+        }
+        // the waves' counts give each its slots (two sets, so that the next
+        // group's are not written over counts a slower wave still reads)
+        if (lane == 0) L.wcnt[par][wave] = w;
+        __syncthreads();
+        int at = have;
+#pragma unroll
+        for (int x = 0; x < kStBlock / 64; ++x) {
+            const int c = L.wcnt[par][x];
+            at += x < wave ? c : 0;
+            have += c;
+        }
+        par ^= 1;
+        if (w == 0) continue;                   // uniform in the wave
+#pragma unroll
+        for (int j = 0; j < kStPer; ++j) {
+            const bool p = (on >> j) & 1u;
+            const uint64_t m = __ballot(p);
+            if (p) {
+                const int o = at + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+                L.d[o] = v[j];
+                L.i[o] = id[j];
+            }
+            at += __builtin_popcountll(m);
+        }
+    }
+    __syncthreads();
+    if (!JOIN && parts > 1) {
+        float* at = row + c0;
+        for (int e = tid; e < E; e += kStBlock) {
+            at[e] = L.d[e];
+            reinterpret_cast<int*>(at + E)[e] = L.i[e];
+        }
+        return;
+    }
+    // sort the E best by (distance, index)
+    if (E <= 64) {
+        if (tid >= 64) return;
+        float d = lane < E ? L.d[lane] : pad_d();
+        int id = lane < E ? L.i[lane] : INT32_MAX;
+        wave_sort(d, id);
+        if (lane < E) {
+            oi[lane] = id;
+            if (od) od[lane] = d;
+        }
+        return;
+    }
+    int n = 128;
+    while (n < E) n <<= 1;                      // n <= 2048 < kStBuf
+    for (int i = E + tid; i < n; i += kStBlock) { L.d[i] = pad_d(); L.i[i] = INT32_MAX; }
+    __syncthreads();
+    for (int size = 2; size <= n; size <<= 1)
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = threadIdx.x; i < n; i += kTopBlock) {
+            for (int i = tid; i < n; i += kStBlock) {
                 const int j = i ^ stride;
                 if (j > i) {
-                    const bool up = ((i & size) == 0);
-                    if (up != lt(sd[i], si[i], sd[j], si[j])) {
-                        const float td = sd[i]; sd[i] = sd[j]; sd[j] = td;
-                        const int ti = si[i]; si[i] = si[j]; si[j] = ti;
+                    const bool up = (i & size) == 0;
+                    if (up != lt(L.d[i], L.i[i], L.d[j], L.i[j])) {
+                        const float td = L.d[i]; L.d[i] = L.d[j]; L.d[j] = td;
+                        const int ti = L.i[i]; L.i[i] = L.i[j]; L.i[j] = ti;
                     }
                 }
             }
             __syncthreads();
         }
+    for (int e = tid; e < E; e += kStBlock) {
+        oi[e] = L.i[e];
+        if (od) od[e] = L.d[e];
     }
 }
 
-// Row top-E of Dm [M, N]: out_idx/out_dist [M, E], ascending by (d, index).
-__global__ __launch_bounds__(kTopBlock) void row_topk(const float* __restrict__ Dm, int64_t M,
-                                                     int64_t N, int E, int32_t* __restrict__ oi,
-                                                     float* __restrict__ od) {
-    __shared__ float sd[kTopBuf];
-    __shared__ int si[kTopBuf];
+__global__ __launch_bounds__(kStBlock, 4) void row_topk_stream(float* __restrict__ Dm, int64_t N,
+                                                            int E, int parts,
+                                                            int32_t* __restrict__ oi,
+                                                            float* __restrict__ od) {
+    const int64_t r = blockIdx.x / parts;
+    const int part = (int)(blockIdx.x - r * parts);
+    row_topk_body<false>(Dm + r * N, N, E, parts, part, oi + r * E, od ? od + r * E : nullptr);
+}
+
+__global__ __launch_bounds__(kStBlock, 4) void row_topk_join(float* __restrict__ Dm, int64_t N, int E,
+                                                          int parts, int32_t* __restrict__ oi,
+                                                          float* __restrict__ od) {
     const int64_t r = blockIdx.x;
-    const float* row = Dm + r * N;
-    int keep = 0;                       // running best held in [0, keep)
-    int64_t c0 = 0;
-    while (c0 < N) {
-        const int64_t take = (N - c0) < (int64_t)(kTopBuf - keep) ? (N - c0) : (kTopBuf - keep);
-        int fill = keep + (int)take;
-        int n = 2;
-        while (n < fill) n <<= 1;
-        for (int i = keep + threadIdx.x; i < n; i += kTopBlock) {
-            const int64_t c = c0 + (i - keep);
-            const bool real = i < fill;
-            sd[i] = real ? row[c] : pad_d();
-            si[i] = real ? (int)c : INT32_MAX;
-        }
-        __syncthreads();
-        lds_sort(sd, si, n);
-        c0 += take;
-        keep = fill < E ? fill : E;
-    }
-    for (int e = threadIdx.x; e < E; e += kTopBlock) {
-        const bool ok = e < keep;
-        oi[r * E + e] = ok ? si[e] : -1;
-        if (od) od[r * E + e] = ok ? sd[e] : INFINITY;
-    }
+    row_topk_body<true>(Dm + r * N, N, E, parts, 0, oi + r * E, od ? od + r * E : nullptr);
+}
+
+// Parts a row of the streaming top-E is read in: enough workgroups for a few
+// on every CU, none shorter than 16,384 columns (eight steps) or 4 E.
+int topk_parts(int64_t nq, int64_t N, int E) {
+    const int64_t shortest = 4 * (int64_t)E > 16384 ? 4 * (int64_t)E : 16384;
+    int64_t p = (1536 + nq - 1) / nq;
+    if (nq >= 512) p = 1;
+    if (p > N / shortest) p = N / shortest;
+    return (int)(p < 1 ? 1 : p > 64 ? 64 : p);
 }
 
 }  // namespace
@@ -616,9 +869,14 @@ static int select_run(const float* Q, int64_t nq, int dim, const float* Vp, int6
     if (P <= (int64_t)kRadBlock * kRadPer && E <= kRadMaxE)
         hipLaunchKernelGGL(row_topk_radix, dim3((unsigned)nq), dim3(kRadBlock), 0, st, Dm, P, E,
                            out_idx, out_dist);
-    else
-        hipLaunchKernelGGL(row_topk, dim3((unsigned)nq), dim3(kTopBlock), 0, st, Dm, nq, P, E,
-                           out_idx, out_dist);
+    else {
+        const int parts = topk_parts(nq, P, E);
+        hipLaunchKernelGGL(row_topk_stream, dim3((unsigned)(nq * parts)), dim3(kStBlock), 0, st,
+                           Dm, P, E, parts, out_idx, out_dist);
+        if (parts > 1)
+            hipLaunchKernelGGL(row_topk_join, dim3((unsigned)nq), dim3(kStBlock), 0, st, Dm, P, E,
+                               parts, out_idx, out_dist);
+    }
     return launch_status("select top-E");
 }
 

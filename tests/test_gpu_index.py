@@ -838,3 +838,38 @@ def test_mfma_probe_reports_a_rate_below_the_published_peak():
     rate = bench.mfma_probe(torch.device("cuda:0"), seconds=0.05)
     note("mfma probe TFLOP/s", rate / 1e12)
     assert 0.2e15 < rate < bench.MFMA_F16_PEAK
+
+
+@pytest.mark.parametrize("nq,P,E", [(1, 16385, 1), (9, 20000, 65), (20, 40960, 2048),
+                                    (513, 16385, 10), (600, 33000, 2048), (12, 400001, 100)])
+@pytest.mark.parametrize("rows", ["random", "descending", "ties", "nan"])
+def test_streamed_top_e_is_the_stable_sort(nq, P, E, rows):
+    """The top-E of rows past 16,384 columns, one part a row and several: exactly
+    the first E of a stable sort (ties to the lower index, NaN last), indices and
+    distances.  With d = 1 and queries of +-1 every distance 1 - q v is one
+    exact product and one rounding, so the reference has the same bits."""
+    from swann_amd import _lib
+    g = torch.Generator().manual_seed(P + E)
+    V = {"random": lambda: torch.randn((P, 1), generator=g),
+         "descending": lambda: torch.linspace(-1, 1, P)[:, None],
+         "ties": lambda: torch.randint(0, 7, (P, 1), generator=g).float(),
+         "nan": lambda: torch.randn((P, 1), generator=g)}[rows]().contiguous()
+    if rows == "nan":
+        V[torch.randint(0, P, (P // 2,), generator=g)] = float("nan")
+    Q = torch.ones((nq, 1))
+    Q[0] = -1
+    Qg, Vg = Q.cuda(), V.cuda()
+    L = _lib.lib()
+    ws = torch.empty(int(L.swann_select_workspace_size(nq, P)), dtype=torch.uint8, device="cuda")
+    idx = torch.empty((nq, E), dtype=torch.int32, device="cuda")
+    dist = torch.empty((nq, E), device="cuda")
+    _lib.call("swann_select_nearest", _lib.ptr(Qg), nq, 1, _lib.ptr(Vg), P, E, 0, _lib.ptr(idx),
+              _lib.ptr(dist), _lib.ptr(ws), _lib.stream_of(Qg.device))
+    # two distinct rows of distances only
+    for q in ([0] if nq == 1 else [0, nq - 1]):
+        d, i = torch.sort(1 - Q[q] * V[:, 0], stable=True)
+        assert torch.equal(idx[q].cpu().long(), i[:E]), (q,)
+        assert torch.equal(torch.nan_to_num(dist[q].cpu(), nan=9e9),
+                           torch.nan_to_num(d[:E], nan=9e9))
+    if nq > 2:
+        assert (idx[1:] == idx[1]).all()
