@@ -28,7 +28,7 @@
 namespace swann {
 namespace {
 
-constexpr int kTM = 64, kTN = 64, kTK = 16;   // GEMM tile
+constexpr int kTM = 64, kTN = 64;             // the tile that the K split is sized by
 constexpr int kTopBuf = 4096;                 // twice the largest E
 constexpr int kRadBlock = 1024, kRadPer = 16; // radix top-E: rows of up to 16384
 constexpr int kRadMaxE = 2048;
@@ -76,62 +76,165 @@ __global__ __launch_bounds__(256) void row_norms(const float* __restrict__ A, in
     if (lane == 0) out[r] = s;
 }
 
-// D[m, n] = f(<A_m, B_n>) for A [M, dim], B [N, dim], both row-major.  With
-// `kper` < dim, workgroup z covers k in [z*kper, (z+1)*kper) and writes the
-// raw partial dot product to Dm + z*M*N (finished by split_finish).
+// D[m, n] = f(<A_m, B_n>) for A [M, dim], B [N, dim], both row-major fp32, on
+// the fp32 matrix cores (32x32x2: fp32 products and sums, a fused
+// multiply-add a term as the vector unit's).  With `kper` < dim, workgroup z
+// covers k in [z*kper, (z+1)*kper) and writes the raw partial dot product to
+// Dm + z*M*N (finished by split_finish).
+//
+// What bounds it is the fp32 MFMA rate (a large library product reaches 154
+// TFLOP/s on this card).  Four waves share a T x T tile, each a quarter of it in
+// 32 x 32 blocks; K advances 32 floats (128 bytes a row) a stage through two LDS
+// buffers, with the loads of two stages ahead in flight in registers.  Chunk c
+// of row r sits at chunk c ^ gswz(r), so the 32 rows of a fragment read fall in
+// distinct banks.  In step t lane l reads chunk 2t + l/32 of its row, four
+// consecutive k, and feeds them to four MFMAs (k = 4 (l/32) + s of the step's 8:
+// a permutation of the order in which a step's terms enter the sum, the same
+// for every row and column, so equal rows have equal distances to the bit).
+// 2,000 x 131,072 x 1,024: 4.3 ms, 125 TFLOP/s (64 x 64 tiles on the vector
+// unit: 15.3 ms); 500 x 4,096 x 960: 50 against 162 us; 4,096 x 4,096 x 1,536:
+// 0.49 against 1.50 ms.
+// T = 128 reads each operand half as often from L2 as T = 64, and is taken once
+// its tiles give every CU two workgroups; below that the smaller tiles keep
+// more of the chip busy.
+// The vector path of the loads (VEC) needs rows of whole 16-byte chunks on a
+// 16-byte boundary; otherwise element loads fill the same stages.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kGK = 32;                        // floats of K a stage
+constexpr int kGRow = kGK * 4;                 // bytes of a row a stage
+
+__device__ __forceinline__ int gswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+template <int T, bool VEC>
 __global__ __launch_bounds__(256) void dist_gemm(const float* __restrict__ A,
                                                  const float* __restrict__ B, int64_t M, int64_t N,
                                                  int dim, int metric,
                                                  const float* __restrict__ an,
                                                  const float* __restrict__ bn,
                                                  float* __restrict__ Dm, int kper) {
-    __shared__ float As[kTK][kTM + 4];
-    __shared__ float Bs[kTK][kTN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;           // 16 x 16 threads, 4 x 4 outputs each
-    const int64_t m0 = (int64_t)blockIdx.y * kTM, n0 = (int64_t)blockIdx.x * kTN;
-    float acc[4][4] = {};
-    // loader: 256 threads x 4 elements = one 64 x 16 tile
-    const int lr = tid >> 2, lk = (tid & 3) * 4;
+    constexpr int BI = T / 64;                 // 32 x 32 blocks a wave, each way
+    constexpr int NL = T / 32;                 // 16-byte chunks a thread stages, each operand
+    __shared__ __align__(16) unsigned char sA[2][T * kGRow];
+    __shared__ __align__(16) unsigned char sB[2][T * kGRow];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+    const int half = lane >> 5;
+    // consecutive tiles of one XCD share their columns' rows (m runs fastest)
+    const int64_t mt = (M + T - 1) / T;
+    const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t m0 = (id % mt) * T, n0 = (id / mt) * T;
     const int kb = blockIdx.z * kper;
     const int ke = (kb + kper < dim) ? kb + kper : dim;
-    for (int k0 = kb; k0 < ke; k0 += kTK) {
+    f32x16 acc[BI][BI];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = k0 + lk + e;
-            const int64_t am = m0 + lr, bnn = n0 + lr;
-            As[lk + e][lr] = (am < M && k < ke) ? A[am * dim + k] : 0.f;
-            Bs[lk + e][lr] = (bnn < N && k < ke) ? B[bnn * dim + k] : 0.f;
-        }
-        __syncthreads();
+    for (int i = 0; i < BI; ++i)
 #pragma unroll
-        for (int k = 0; k < kTK; ++k) {
-            float a[4], b[4];
+        for (int j = 0; j < BI; ++j) acc[i][j] = (f32x16){};
+    // rows past the matrix read its last row; their sums are not written
+    const float* pa[NL];
+    const float* pb[NL];
+    int lds[NL];
+    const int ch = tid & 7;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[k][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
+    for (int q = 0; q < NL; ++q) {
+        const int r = q * 32 + (tid >> 3);
+        pa[q] = A + (m0 + r < M ? m0 + r : M - 1) * dim;
+        pb[q] = B + (n0 + r < N ? n0 + r : N - 1) * dim;
+        lds[q] = r * kGRow + ((ch ^ gswz(r)) << 4);
     }
+    // every load is issued, past the end of K from the row's first chunk, and
+    // zeroed at staging: no branch for the loads in flight to be waited at
+    f32x4 ra[NL], rb[NL];
+    int left = 0;                              // elements of the fetched chunk inside K
+    auto fetch = [&](int k0) {
+        const int k = k0 + ch * 4;
+        left = ke - k;
+        const int kc = left > 0 ? k : kb;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t m = m0 + ty * 4 + i;
-        if (m >= M) continue;
+        for (int q = 0; q < NL; ++q) {
+            if constexpr (VEC) {
+                ra[q] = *reinterpret_cast<const f32x4*>(pa[q] + kc);
+                rb[q] = *reinterpret_cast<const f32x4*>(pb[q] + kc);
+            } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t nn = n0 + tx * 4 + j;
-            if (nn >= N) continue;
-            const float s = acc[i][j];
-            if (kper < dim)
-                Dm[(int64_t)blockIdx.z * M * N + m * N + nn] = s;
-            else
-                Dm[m * N + nn] = metric == SWANN_METRIC_IP ? 1.0f - s : (bn[nn] - 2.0f * s) + an[m];
+                for (int e = 0; e < 4; ++e) {
+                    const int ke1 = e < left ? kc + e : kb;
+                    ra[q][e] = pa[q][ke1];
+                    rb[q][e] = pb[q][ke1];
+                }
+            }
         }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            f32x4 va = ra[q], vb = rb[q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                va[e] = (VEC ? 0 : e) < left ? va[e] : 0.f;
+                vb[e] = (VEC ? 0 : e) < left ? vb[e] : 0.f;
+            }
+            *reinterpret_cast<f32x4*>(&sA[buf][lds[q]]) = va;
+            *reinterpret_cast<f32x4*>(&sB[buf][lds[q]]) = vb;
+        }
+    };
+    const int fsw = gswz(lane & 31);           // fragment rows are 32 x + lane % 32
+    fetch(kb);
+    stage(0);
+    fetch(kb + kGK);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = kb; k0 < ke; k0 += kGK) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            // half way, the next stage goes to the other buffer (last read
+            // before the barrier this stage began at) and the one after it is
+            // fetched: both among the MFMAs, so the waves of a CU do not meet
+            // at the stage's end with nothing to multiply
+            if (t == 2) {
+                stage(buf ^ 1);
+                fetch(k0 + 2 * kGK);
+            }
+            const int co = ((2 * t + half) ^ fsw) << 4;
+            f32x4 fa[BI], fb[BI];
+#pragma unroll
+            for (int i = 0; i < BI; ++i) {
+                const int r = i * 32 + (lane & 31);
+                fa[i] = *reinterpret_cast<const f32x4*>(&sA[buf][(wm + r) * kGRow + co]);
+                fb[i] = *reinterpret_cast<const f32x4*>(&sB[buf][(wn + r) * kGRow + co]);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < BI; ++i)
+#pragma unroll
+                    for (int j = 0; j < BI; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][s], fb[j][s],
+                                                                         acc[i][j], 0, 0, 0);
+        }
+        __syncthreads();
+        buf ^= 1;
+    }
+    // lane: column lane % 32 of a block, rows (e / 4) * 8 + 4 (lane / 32) + e % 4
+#pragma unroll
+    for (int j = 0; j < BI; ++j) {
+        const int64_t nn = n0 + wn + j * 32 + (lane & 31);
+        if (nn >= N) continue;
+        const float b = metric == SWANN_METRIC_L2 && kper >= dim ? bn[nn] : 0.f;
+#pragma unroll
+        for (int i = 0; i < BI; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int64_t m = m0 + wm + i * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
+                if (m >= M) continue;
+                const float s = acc[i][j][e];
+                if (kper < dim)
+                    Dm[(int64_t)blockIdx.z * M * N + m * N + nn] = s;
+                else
+                    Dm[m * N + nn] = metric == SWANN_METRIC_IP ? 1.0f - s : (b - 2.0f * s) + an[m];
+            }
     }
 }
 
@@ -825,20 +928,24 @@ static int gemm_run(const float* Q, int64_t nq, int dim, const float* Vp, int64_
     int kper = dim;
     if (S > 1) {
         kper = (dim + S - 1) / S;
-        kper = ((kper + kTK - 1) / kTK) * kTK;
+        kper = ((kper + 15) / 16) * 16;
         S = (dim + kper - 1) / kper;
     }
-    dim3 grid((unsigned)((P + kTN - 1) / kTN), (unsigned)((nq + kTM - 1) / kTM), (unsigned)S);
-    if (S > 1) {
-        float* part = (float*)((char*)vn + ((P * 4 + 255) / 256) * 256);
-        hipLaunchKernelGGL(dist_gemm, grid, dim3(256), 0, st, Q, Vp, nq, P, dim, metric, qn, vn,
-                           part, kper);
+    float* out = Dm;
+    if (S > 1) out = (float*)((char*)vn + ((P * 4 + 255) / 256) * 256);
+    else kper = dim;
+    // 128 x 128 tiles once they give every CU two workgroups
+    const bool vec = dim % 4 == 0 && (uintptr_t)Q % 16 == 0 && (uintptr_t)Vp % 16 == 0;
+    const bool big = ((P + 127) / 128) * ((nq + 127) / 128) >= 512;
+    const int T = big ? 128 : 64;
+    const dim3 grid((unsigned)(((P + T - 1) / T) * ((nq + T - 1) / T)), 1, (unsigned)S);
+    auto* kernel = big ? (vec ? dist_gemm<128, true> : dist_gemm<128, false>)
+                       : (vec ? dist_gemm<64, true> : dist_gemm<64, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, Q, Vp, nq, P, dim, metric, qn, vn, out,
+                       kper);
+    if (S > 1)
         hipLaunchKernelGGL(split_finish, dim3((unsigned)((nq * P + 255) / 256)), dim3(256), 0, st,
-                           part, S, nq, P, metric, qn, vn, Dm);
-    } else {
-        hipLaunchKernelGGL(dist_gemm, grid, dim3(256), 0, st, Q, Vp, nq, P, dim, metric, qn, vn,
-                           Dm, dim);
-    }
+                           out, S, nq, P, metric, qn, vn, Dm);
     return launch_status("select gemm");
 }
 

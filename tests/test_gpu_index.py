@@ -873,3 +873,39 @@ def test_streamed_top_e_is_the_stable_sort(nq, P, E, rows):
                            torch.nan_to_num(d[:E], nan=9e9))
     if nq > 2:
         assert (idx[1:] == idx[1]).all()
+
+
+@pytest.mark.parametrize("nq,P,d", [(9, 16, 1), (64, 65, 31), (65, 1000, 33), (300, 4097, 100),
+                                    (1025, 8193, 40), (1100, 7680, 65)])
+@pytest.mark.parametrize("metric", [0, 1])
+def test_selection_distances_are_fp32_sums(nq, P, d, metric):
+    """The distance product at the edges of its tiles (64 and 128 rows and
+    columns, 32 of K, widths that are no multiple of 4, the K split of small
+    grids): every distance within the rounding of an fp32 sum of `d` products,
+    d u sum |q v| (u = 2^-24, and the few roundings of the formula), of the
+    float64 one."""
+    from swann_amd import _lib
+    g = torch.Generator().manual_seed(nq + d)
+    Q, V = torch.randn((nq, d), generator=g), torch.randn((P, d), generator=g)
+    E = min(P, 64)
+    Qg, Vg = Q.cuda(), V.cuda()
+    ws = torch.empty(int(_lib.lib().swann_select_workspace_size(nq, P)), dtype=torch.uint8,
+                     device="cuda")
+    idx = torch.empty((nq, E), dtype=torch.int32, device="cuda")
+    dist = torch.empty((nq, E), device="cuda")
+    _lib.call("swann_select_nearest", _lib.ptr(Qg), nq, d, _lib.ptr(Vg), P, E, metric,
+              _lib.ptr(idx), _lib.ptr(dist), _lib.ptr(ws), _lib.stream_of(Qg.device))
+    q, v = Q.double(), V.double()
+    dot, mag = q @ v.T, q.abs() @ v.abs().T
+    qq, vv = (q * q).sum(1)[:, None], (v * v).sum(1)[None, :]
+    D = 1 - dot if metric == 0 else vv - 2 * dot + qq
+    u = 2.0 ** -24
+    bound = ((d + 2) * u * mag + 2 * u * (1 + dot.abs()) if metric == 0 else
+             (2 * d + 6) * u * mag + (d + 6) * u * (qq + vv))
+    got = idx.cpu().long()
+    err = (dist.cpu().double() - D.gather(1, got)).abs()
+    assert (err <= bound.gather(1, got)).all()
+    # and they are the E nearest, up to that bound
+    kth = torch.topk(D, E, dim=1, largest=False).values[:, -1]
+    assert (D.gather(1, got).max(1).values <= kth + 2 * bound.max(1).values).all()
+    assert (dist.cpu().diff(dim=1) >= 0).all()
