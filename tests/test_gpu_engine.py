@@ -792,3 +792,28 @@ def test_branches_spread_over_xcds_match_oracle(opt):
         for j in range(0, J, 5):
             br = O.run(X, G, Qv[qi], int(seeds[qi, j]), L=12, B=30, team=16, stop_eps=0.05)
             assert_queue(st, qi, j, br, (qi, j))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("n,d", [(1, 1), (7, 31), (33, 64), (40, 100), (300, 520), (1025, 513),
+                                 (2000, 1032)])
+def test_build_codes_at_row_and_word_edges(n, d, dtype):
+    """Codes of rows that fill no whole chunk, word, group of columns or workgroup,
+    and of rows that start off a 16-byte boundary: the float64 means and scales to
+    a rounding, the bits exactly."""
+    from swann_amd.codes import build_codes
+    g = torch.Generator().manual_seed(n + d)
+    X = torch.randn((n, d), generator=g).to(torch.float32 if dtype == "f32" else torch.float16)
+    for off in (0, 1):
+        buf = torch.zeros(n * d + 1, dtype=X.dtype, device="cuda")
+        Xg = buf[off:off + n * d].view(n, d)
+        Xg.copy_(X)
+        codes, alpha, mu = (t.cpu() for t in build_codes(Xg))
+        want = X.double().mean(0).float()
+        assert torch.allclose(mu, want, rtol=2.0 ** -23, atol=1e-12)
+        df = X.float() - mu
+        bits = torch.zeros((n, codes.shape[1] * 32), dtype=torch.int64)
+        bits[:, :d] = (df > 0)
+        words = (bits.view(n, -1, 32) << torch.arange(32)).sum(2)
+        assert torch.equal(codes.long() & 0xFFFFFFFF, words)
+        assert torch.allclose(alpha, df.double().abs().mean(1).float(), rtol=2.0 ** -23)
