@@ -18,6 +18,7 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -212,6 +213,12 @@ struct MfmaSweepArgs {
     // cannot take the row for unchanged (sym_merge)
     int* mcnt;
     int tstride;                 // the bounded repair's list stride (tiles a panel)
+    // symmetric sweep around the circle (0: the triangle): panel I takes tiles
+    // (I, (I + b) mod ntile) for b in [b0, b1), every panel the same number, and
+    // `wrap` workgroups share a panel's, each a run of its offsets.  The first
+    // keeps list 0; the others append what they find for the panel's own rows
+    // to list 1, as any workgroup does for its column panels' rows.
+    int wrap;
 };
 
 // Wave-cooperative compaction of one row's buffer to its C best (exact:
@@ -315,6 +322,28 @@ __device__ __forceinline__ float screen_thr(float thr, float na) {
     return 0.5f * ((na - thr) - 1e-5f * (fabsf(na) + fabsf(thr)));
 }
 
+// A survivor for row `row`'s second list, of candidate `id` at distance d: queued
+// in LDS as entry x, or, past the queue's end or without one, appended at once.
+constexpr int kFQueue = 1024;
+constexpr int kFOwn = 1 << 30;
+
+__device__ __forceinline__ void push_second(const MfmaSweepArgs& a, bool fstage, int* qn, int2* qe,
+                                            int x, float d, int64_t row, int64_t id) {
+    const int k = fstage ? atomicAdd(qn, 1) : kFQueue;
+    if (k < kFQueue) {
+        qe[k] = make_int2(x, __float_as_int(d));
+        return;
+    }
+    const int p = atomicAdd(&a.bcnt[row * 2 + 1], 1);
+    if (p < a.fcap) {
+        const int64_t o = (row * 2 + 1) * (int64_t)a.cap + p;
+        a.bkey[o] = d;
+        a.bid[o] = (int32_t)id;
+    } else {
+        atomicAdd(a.ovf, 1);
+    }
+}
+
 // Epilogue for one 32 x 32 accumulator block: lane holds column c and the 16
 // rows rbase + (e/4)*8 + (e%4).  The common case -- no score of the block
 // beats its row's threshold -- costs the distance formula and one compare per
@@ -328,12 +357,14 @@ __device__ __forceinline__ float screen_thr(float thr, float na) {
 // recomputed exactly from fresh LDS reads and appended to its row's buffer.
 // Called by the lanes whose screen passed, once the wave's ballot has shown
 // that some did.
-template <int METRIC>
+template <int METRIC, bool SHARE = false>
 __device__ __forceinline__ void append_own(const f32x16& v, int rbase, int64_t r0, int64_t c,
                                            float cn, float sc, const float* rs, const float* thr,
                                            const float* rnorm, int* cnt, const MfmaSweepArgs& a,
                                            int split, int nterm_scale, const f32x16* vx,
-                                           int* needf, bool cok = true) {
+                                           int* needf, bool cok = true, bool shared = false,
+                                           bool fstage = false, int cl = 0, int* qn = nullptr,
+                                           int2* qe = nullptr) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const float4 t4 = *reinterpret_cast<const float4*>(thr + rbase + g * 8);
@@ -356,6 +387,10 @@ __device__ __forceinline__ void append_own(const f32x16& v, int rbase, int64_t r
             const float d = dist_formula<METRIC>(dot, METRIC == SWANN_METRIC_L2 ? r4[q] : 0.f, cn);
             if (!(d < t4[q])) continue;
             const int rl = rbase + g * 8 + q;
+            if (SHARE && shared) {
+                push_second(a, fstage, qn, qe, kFOwn | (cl << 16) | rl, d, r0 + rl, c);
+                continue;
+            }
             const int p = atomicAdd(&cnt[rl], 1);
             // the append that leaves less than a tile of room flags a compaction
             if (needf && p == a.cap - kBN2) *needf = 1;
@@ -428,57 +463,22 @@ __device__ __forceinline__ void epilogue_block(const f32x16& v, int rbase, int64
 // of the column panel, whose threshold `thc` came from the last merge -- and
 // its 16 candidates rbase + (e/4)*8 + (e%4) of the row panel.  Row c's
 // distance to candidate r is the reference formula with the roles swapped
-// (na = |c|^2, nb = |r|^2), from the same score.  Survivors of the screen
-// (screen_pair) take a slot of row c's second list from its global counter.
-// Candidates past n are copies of row n - 1 (the panel loads clamp) and are
-// skipped.
-template <int METRIC>
-__device__ __forceinline__ void append_foreign(const f32x16& v, int rbase, int64_t r0,
-                                               int64_t c, float cn, float sc, float thc,
-                                               const float* rs, const float* rnorm,
-                                               const MfmaSweepArgs& a, int scaled, bool cok) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const float4 s4 = scaled ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
-                                 : make_float4(1.f, 1.f, 1.f, 1.f);
-        const float4 r4 = METRIC == SWANN_METRIC_L2
-                              ? *reinterpret_cast<const float4*>(rnorm + rbase + g * 8)
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float dot = scaled ? s4[q] * sc * v[g * 4 + q] : v[g * 4 + q];
-            if (!cok) continue;
-            const float d = dist_formula<METRIC>(dot, cn, r4[q]);
-            const int64_t r = r0 + rbase + g * 8 + q;
-            if (!(d < thc) || r >= a.n) continue;
-            const int p = atomicAdd(&a.bcnt[c * 2 + 1], 1);
-            if (p < a.fcap) {
-                const int64_t o = (c * 2 + 1) * (int64_t)a.cap + p;
-                a.bkey[o] = d;
-                a.bid[o] = (int32_t)r;
-            } else {
-                atomicAdd(a.ovf, 1);
-            }
-        }
-    }
-}
-
-// Foreign survivors queued in LDS instead of taking their global slots at
-// once: a slot is a returning atomic on row c's counter, and a wave that
-// waits for it (vmcnt) stalls for a memory round trip per survivor.  The
-// queue (column and row within the tile, distance) is drained at the next
-// column tile's first stage, where each thread takes one entry's slot with
-// an atomic whose return is waited for by that stage's own barrier, and the
-// entries are stored at the second stage.  A full queue takes the direct
-// path.
-constexpr int kFQueue = 1024;
-
+// (na = |c|^2, nb = |r|^2), from the same score.  Candidates past n are copies
+// of row n - 1 (the panel loads clamp) and are skipped.
+//
+// Survivors are queued in LDS (push_second) instead of taking their slots of
+// row c's second list at once: a slot is a returning atomic on the row's
+// global counter, and a wave that waits for it (vmcnt) stalls for a memory
+// round trip per survivor.  The queue (column and row within the tile, kFOwn,
+// distance) is drained at the next column tile's first stage, where each thread
+// takes one entry's slot with an atomic whose return is waited for by that
+// stage's own barrier, and the entries are stored at the second stage.
 template <int METRIC>
 __device__ __forceinline__ void queue_foreign(const f32x16& v, int rbase, int64_t r0, int64_t c,
                                               int cl, float cn, float sc, float thc,
                                               const float* rs, const float* rnorm,
-                                              const MfmaSweepArgs& a, int scaled, int* qn,
-                                              int2* qe, bool cok) {
+                                              const MfmaSweepArgs& a, int scaled, bool fstage,
+                                              int* qn, int2* qe, bool cok) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const float4 s4 = scaled ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
@@ -493,21 +493,16 @@ __device__ __forceinline__ void queue_foreign(const f32x16& v, int rbase, int64_
             const float d = dist_formula<METRIC>(dot, cn, r4[q]);
             const int rl = rbase + g * 8 + q;
             if (!(d < thc) || r0 + rl >= a.n) continue;
-            const int k = atomicAdd(qn, 1);
-            if (k < kFQueue) {
-                qe[k] = make_int2((cl << 16) | rl, __float_as_int(d));
-            } else {
-                const int p = atomicAdd(&a.bcnt[c * 2 + 1], 1);
-                if (p < a.fcap) {
-                    const int64_t o = (c * 2 + 1) * (int64_t)a.cap + p;
-                    a.bkey[o] = d;
-                    a.bid[o] = (int32_t)(r0 + rl);
-                } else {
-                    atomicAdd(a.ovf, 1);
-                }
-            }
+            push_second(a, fstage, qn, qe, (cl << 16) | rl, d, c, r0 + rl);
         }
     }
+}
+
+// A queued entry's row and candidate, from its tile's row and column bases.
+struct Queued { int row, id; };
+__device__ __forceinline__ Queued queued(int x, int r0, int cb) {
+    const int r = r0 + (x & 0xffff), c = cb + ((x >> 16) & 0x3fff);
+    return (x & kFOwn) ? Queued{r, c} : Queued{c, r};
 }
 
 // Both screens of a block of the DMA sweep in one pass, as wave masks: each
@@ -763,6 +758,15 @@ constexpr int kStage = kBM2 * kRowBytes;           // 32 KB per operand per stag
 
 typedef __attribute__((address_space(3))) void* lds_vptr;
 
+// f(integral_constant<0>) .. f(integral_constant<N - 1>)
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 // One wave-wide direct load global -> LDS of 16 bytes a lane: lane i's 16
@@ -817,9 +821,14 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     // symmetric sweep: the current column tile's rows' thresholds (from the
     // last merge, fixed for the launch), for the foreign half of its epilogue
     __shared__ __align__(16) float thrc[kBN2];
-    // symmetric sweep: foreign survivors waiting for their slots (queue_foreign)
+    // symmetric sweep: second-list survivors waiting for their slots (push_second)
     __shared__ int fqn;
     __shared__ int2 fq[kFQueue];
+    // scalars that only a tile's start or an append reads, kept out of the
+    // stages' registers (held, they spill, and a reload waits for the direct
+    // loads): first column tile, its place in the order, offsets or 0 (in
+    // order), column tiles; whether another workgroup keeps list 0
+    __shared__ int run[5];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -837,7 +846,11 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     // symmetric sweep: one workgroup per row panel, which keeps list 0 of
     // its rows and starts from the thresholds and lists the last merge left;
     // sym_panel spreads the band's short panels over the XCDs
-    const int lid = a.sym ? sym_panel((int)blockIdx.x, (int)gridDim.x, (int)(a.b1 - a.b0))
+    // around the circle, consecutive panels of one run of offsets share an XCD
+    const int wid = a.wrap ? (int)xcd_remap(blockIdx.x, gridDim.x) : 0;
+    const int sub = a.wrap ? wid / ntile : 0;
+    const int lid = a.wrap ? wid - sub * ntile
+                  : a.sym ? sym_panel((int)blockIdx.x, (int)gridDim.x, (int)(a.b1 - a.b0))
                           : (int)xcd_remap(blockIdx.x, (int64_t)(a.plist ? a.npl : ntile) * G);
     const int r0 = (a.sym ? lid : a.plist ? a.plist[lid / G] : lid / G) * kBM2;
     const int split = a.sym ? 0 : lid % G;
@@ -864,6 +877,14 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     if (a.sym) {
         ct0 = lid + (int)a.b0;
         ct1 = lid + a.b1 < nct ? lid + (int)a.b1 : nct;
+    }
+    int bw = a.sym ? (int)(a.b1 - a.b0) : 0;       // offsets of this workgroup's run
+    if (a.wrap) {
+        const int o0 = (int)a.b0 + bw * sub / a.wrap, o1 = (int)a.b0 + bw * (sub + 1) / a.wrap;
+        bw = o1 - o0;
+        ct0 = lid + o0;
+        // half way round an even circle, (I, J) and (J, I) meet: the lower scores it
+        ct1 = lid + o1 - (2 * (o1 - 1) == ntile && 2 * lid >= ntile ? 1 : 0);
     }
     // with a tile list the column tiles are a listed subset, in order: in a
     // symmetric launch (the pruned ordered sweep) panel lid's, inside its
@@ -927,13 +948,22 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     // lines in L2; in the order ct0 + k, neighbours read the same panel one
     // tile apart, long after L2 has dropped it.  The lists do not depend on
     // the order.
-    const int bw = a.sym ? (int)(a.b1 - a.b0) : 0;
     const bool rot = a.sym && !tls && bw > 1 && ntl == bw;
-    const int cmod = rot ? ct0 % bw : 0;
+    const bool fstage = a.sym && nk >= 3;    // the foreign queue (below)
+    if (tid == 0) {
+        run[0] = ct0;
+        run[1] = rot ? ct0 % bw : 0;
+        run[2] = rot ? bw : 0;
+        run[3] = nct;
+        run[4] = sub > 0;                    // another workgroup keeps list 0
+    }
+    __syncthreads();
     auto tile_at = [&](int k) {
         if (tls) return __builtin_amdgcn_readfirstlane(tls[k]);
-        if (rot) return ct0 + (k >= cmod ? k - cmod : k - cmod + bw);
-        return ct0 + k;
+        const int m = run[1];
+        int ct = run[0] + (k >= m ? k - m : k - m + run[2]);
+        ct = ct < run[3] ? ct : ct - run[3];     // past the end: around the circle
+        return __builtin_amdgcn_readfirstlane(ct);
     };
     int kt_c = 0, kt_f = 0, ki_c = 0, ki_f = 0;
     int cb_c = ntl > 0 ? tile_at(0) * kBN2 : 0, cb_f = cb_c;
@@ -947,7 +977,6 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     // the foreign queue: staged when a tile has at least three stages, so
     // that its drain (first stage) and stores (second) come before the next
     // epilogue (last stage) refills it
-    const bool fstage = a.sym && nk >= 3;
     int fslot = 0, fqd = 0;          // this thread's drained entry: its slot; entries drained
     int cb_prev = 0;                 // column base of the tile whose entries are queued
     int tpar = 0;                    // parity of the current column tile (its need flag)
@@ -983,19 +1012,17 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
             // take the slots of the last tile's queued foreign survivors; the
             // returns are waited for by the next stage's barrier
             fqd = fqn < kFQueue ? fqn : kFQueue;
-            if (tid < fqd) {
-                const int2 e = fq[tid];
-                fslot = atomicAdd(&a.bcnt[(int64_t)(cb_prev + (e.x >> 16)) * 2 + 1], 1);
-            }
+            if (tid < fqd)
+                fslot = atomicAdd(&a.bcnt[(int64_t)queued(fq[tid].x, r0, cb_prev).row * 2 + 1], 1);
         }
         if (fstage && kt == 1) {
             if (tid < fqd) {
                 const int2 e = fq[tid];
-                const int64_t c = cb_prev + (e.x >> 16);
+                const Queued w = queued(e.x, r0, cb_prev);
                 if (fslot < a.fcap) {
-                    const int64_t o = (c * 2 + 1) * (int64_t)a.cap + fslot;
+                    const int64_t o = ((int64_t)w.row * 2 + 1) * (int64_t)a.cap + fslot;
                     a.bkey[o] = __int_as_float(e.y);
-                    a.bid[o] = (int32_t)(r0 + (e.x & 0xffff));
+                    a.bid[o] = (int32_t)w.id;
                 } else {
                     atomicAdd(a.ovf, 1);
                 }
@@ -1088,12 +1115,14 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
             // ---- epilogue of this column tile: distance, threshold, append ----
             const int cb = cbt;
             const bool diag = (cb == r0);
-#pragma unroll
-            for (int j = 0; j < BJ; ++j) {
+            // unrolled by the template, whatever its size: indexed at run time,
+            // the accumulators would live in scratch memory
+            static_for<BJ>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
                 const int c = cb + wn * CW + j * 32 + (lane & 31);
                 const bool cok = c < n;
-#pragma unroll
-                for (int i = 0; i < BI; ++i) {
+                static_for<BI>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
                     int rbase = wm * RW + i * 32 + (lane >> 5) * 4;
                     asm volatile("" : "+v"(rbase));
                     if (diag) self_out(acc[i][j], rbase, wn * CW + j * 32 + (lane & 31));
@@ -1107,22 +1136,19 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
                     const uint64_t valid = __ballot(cok);
                     if (own & valid) {
                         asm volatile("" ::: "memory");   // rare path: reload, do not keep live
-                        append_own<METRIC>(acc[i][j], rbase, r0, c, cn[j], cs[j], rscale, thr,
-                                           rnorm, cnt, a, split, SCALED ? 2 : 0, nullptr,
-                                           &need[tpar], cok);
+                        append_own<METRIC, true>(acc[i][j], rbase, r0, c, cn[j], cs[j], rscale,
+                                                 thr, rnorm, cnt, a, split, SCALED ? 2 : 0,
+                                                 nullptr, &need[tpar], cok, run[4] != 0, fstage,
+                                                 c - cb, &fqn, fq);
                     }
                     if (frn & valid) {
                         asm volatile("" ::: "memory");
-                        if (fstage)
-                            queue_foreign<METRIC>(acc[i][j], rbase, r0, c, c - cb, cn[j], cs[j],
-                                                  thc, rscale, rnorm, a, SCALED, &fqn, fq, cok);
-                        else
-                            append_foreign<METRIC>(acc[i][j], rbase, r0, c, cn[j], cs[j], thc,
-                                                   rscale, rnorm, a, SCALED, cok);
+                        queue_foreign<METRIC>(acc[i][j], rbase, r0, c, c - cb, cn[j], cs[j], thc,
+                                              rscale, rnorm, a, SCALED, fstage, &fqn, fq, cok);
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+                });
+            });
             tpar ^= 1;
             cb_prev = cb;
         }
@@ -1134,12 +1160,12 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
         const int nq = fqn < kFQueue ? fqn : kFQueue;
         for (int k = tid; k < nq; k += WAVES * 64) {
             const int2 e = fq[k];
-            const int64_t c = cb_prev + (e.x >> 16);
-            const int p = atomicAdd(&a.bcnt[c * 2 + 1], 1);
+            const Queued w = queued(e.x, r0, cb_prev);
+            const int p = atomicAdd(&a.bcnt[(int64_t)w.row * 2 + 1], 1);
             if (p < a.fcap) {
-                const int64_t o = (c * 2 + 1) * (int64_t)a.cap + p;
+                const int64_t o = ((int64_t)w.row * 2 + 1) * (int64_t)a.cap + p;
                 a.bkey[o] = __int_as_float(e.y);
-                a.bid[o] = (int32_t)(r0 + (e.x & 0xffff));
+                a.bid[o] = (int32_t)w.id;
             } else {
                 atomicAdd(a.ovf, 1);
             }
@@ -1156,7 +1182,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
         }
         __syncthreads();
     }
-    if (tid < kBM2 && r0 + tid < n) a.bcnt[(int64_t)(r0 + tid) * G + split] = cnt[tid];
+    if (tid < kBM2 && r0 + tid < n && run[4] == 0)
+        a.bcnt[(int64_t)(r0 + tid) * G + split] = cnt[tid];
 }
 
 // ---------------------------------------------------------------------------
@@ -2199,7 +2226,7 @@ __global__ __launch_bounds__(256) void repair_merge(const float* __restrict__ rk
         const int64_t at = ((int64_t)rl * kRepairSplits + sg) * cap + off;
         sd[i] = real ? rkey[at] : INFINITY;
         si[i] = real ? rid[at] : INT32_MAX;
-        so[i] = real ? perm[rid[at]] : INT32_MAX;    // the order of ties
+        so[i] = real ? (perm ? perm[rid[at]] : rid[at]) : INT32_MAX;   // the order of ties
     }
     __syncthreads();
     for (int size = 2; size <= np; size <<= 1)
@@ -2277,13 +2304,44 @@ inline int64_t band_tiles(int64_t ntile, int64_t b0, int64_t b1) {
     return M <= B ? M * (M + 1) / 2 : B * (B + 1) / 2 + (M - B) * B;
 }
 
-// Whether the direct-load sweep runs symmetric: by default when there are at
-// least 1,024 row panels (n > 261,888), where every band launch still fills
-// the GPU; option sweep_sym = 0|1 forces it.
+// Workgroups that share a panel's band of B offsets in a launch around the
+// circle.  Every panel has the same work there, so a launch takes the rounds of
+// ntile * S workgroups the CUs need, each of ceil(B / S) tiles (and about half a
+// tile of start and end): the S of least cost, preferring the smaller unless a
+// larger saves 3%.  At 391 panels (n = 100,000) one workgroup a panel leaves a
+// second round of 135 on 256 CUs (0.76 of them busy); five are 7.6 rounds of
+// a fifth each (0.95).
+inline int band_shares(int64_t ntile, int64_t B, int cus) {
+    int best = 1;
+    double cost = 0;
+    for (int S = 1; S <= 8 && S <= B; ++S) {
+        const double c = (double)((ntile * S + cus - 1) / cus) * ((double)((B + S - 1) / S) + 0.5);
+        if (S == 1 || c < 0.97 * cost) { best = S; cost = c; }
+    }
+    return best;
+}
+
+// Whether the direct-load sweep runs symmetric: by default from 32 row panels
+// (n > 7,936), below which the launches of its bands cost more than the half of
+// the tiles it leaves out; option sweep_sym = 0|1 forces it.  C = 128, widths 64
+// to 1,536: at 4,500 and 6,000 rows within 10% of the one-sided sweep either way,
+// at 8,000 16 to 28% faster, from 10,000 1.3 to 2 times (100,000 x 1,536 fp16:
+// 50.3 against 24.7 ms).
 inline bool sweep_sym(int64_t ntile) {
     const int f = option(kOptSweepSym);
     if (f >= 0) return f == 1 && ntile >= 2;
-    return ntile >= 1024;
+    return ntile >= 32;
+}
+
+// The symmetric sweep reads its overflow count back, which a stream under graph
+// capture cannot: there the one-sided sweep runs.
+inline bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return c != hipStreamCaptureStatusNone;
 }
 
 // Waves per direct-load workgroup: 16 (64 x 64 wave tiles, the default) or
@@ -2341,7 +2399,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
         hi = h;
     }
     MfmaSweepArgs a{hi, nullptr, scale, xn, n, dim, metric, C, cap, bkey, bid, bcnt, scaled, 1,
-                    0, 0, 0, nullptr, nullptr, cap};
+                    0, 0, 0, nullptr, nullptr, cap};                 // the rest 0
     const unsigned grid = (unsigned)((n + kBM2 - 1) / kBM2);
     const bool ip = metric == SWANN_METRIC_IP;
     *used = 1;
@@ -2349,7 +2407,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
     const bool off32 = (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32);
     if (dim % kBK3 == 0 && (uintptr_t)hi % 16 == 0 && off32 && !option_on(kOptSweepRegstage)) {
         const int64_t ntile = (n + kBM2 - 1) / kBM2;
-        if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16) {
+        if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !capturing(st)) {
             // symmetric sweep: tile (I, J), J >= I, scored once for the rows of
             // both panels; launched in bands of J - I (1, 1, 2, 4, ... 256, then
             // kBandMax at a time) with a merge after each, so every launch
@@ -2387,14 +2445,28 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
             int64_t host_tiles = 0;      // tiles of the launches not pruned
             // the launches of bands [b0, bend), each followed by a merge;
             // with `prune`, each launch scores only the tiles tile_keep keeps
+            int cus = 0, dev = 0;
+            if (hipGetDevice(&dev) != hipSuccess ||
+                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
+                    hipSuccess || cus < 1) {
+                (void)hipGetLastError();
+                cus = 256;
+            }
+            // (without a prune and from the first band: around the circle)
             auto bands = [&](MfmaSweepArgs& sa, int64_t bstart, int64_t bend, const float* seed,
-                             int* flag, bool prune) -> int {
+                             int* flag, bool prune, bool circle = false) -> int {
                 for (int64_t b0 = bstart; b0 < bend;) {
                     const int64_t B = b0 == 0 ? 1 : (b0 < kBandMax ? b0 : kBandMax);
                     sa.b0 = b0;
                     sa.b1 = b0 + B < bend ? b0 + B : bend;
-                    const unsigned grid = (unsigned)(ntile - b0);
-                    if (prune) {
+                    sa.wrap = circle ? band_shares(ntile, sa.b1 - b0, cus) : 0;
+                    const unsigned grid = (unsigned)(circle ? ntile * sa.wrap : ntile - b0);
+                    if (circle) {
+                        sa.tlist = nullptr;
+                        sa.tcnt = nullptr;
+                        host_tiles += ntile * (sa.b1 - b0) -
+                                      (2 * (sa.b1 - 1) == ntile ? ntile / 2 : 0);
+                    } else if (prune) {
                         hipLaunchKernelGGL(panel_thr, dim3((unsigned)ntile), dim3(256), 0, st,
                                            (const float*)gthr, n, (const int*)dns, pthr);
                         hipLaunchKernelGGL(tile_keep, dim3(grid), dim3(64), 0, st, tlb,
@@ -2542,8 +2614,10 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                                        perm);
                 }
                 if (!clustered) {
+                    // not clustered: the rows' own order, no seeds; the flags
+                    // name the rows to repair
                     seed = nullptr;
-                    flag = nullptr;
+                    hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
                     goto plain;
                 }
                 hipLaunchKernelGGL(gather_rows, dim3(nrb), dim3(256), 0, st, hi, n, dim, perm, xn,
@@ -2684,13 +2758,13 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
             hipLaunchKernelGGL(sym_init, dim3(nb256), dim3(256), 0, st, gthr, bcnt, ovf, n,
                                (const float*)seed, mcnt);
             {
-                const int rc = bands(s, 0, ntile, seed, flag, false);
+                const int rc = bands(s, 0, ntile / 2 + 1, seed, flag, false, true);
                 if (rc) return rc;
             }
         swept:
-            // a list that overflowed lost candidates: redo the sweep the
-            // one-sided way (one small read-back; the build is not on the
-            // search path)
+            // a list that overflowed lost candidates: sweep its panel again
+            // the one-sided way, or without flags every panel (one small
+            // read-back; the build is not on the search path)
             int dropped = 0;
             unsigned long long pruned_kept = 0;
             if (hipMemcpyAsync(&dropped, ovf, sizeof(int), hipMemcpyDeviceToHost, st) !=
@@ -2707,8 +2781,8 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                 *perm_out = ordered;
                 return SWANN_OK;
             }
-            if (ordered) {
-                // the ordered sweep's repair: the row panels holding a row
+            if (ordered || flag) {
+                // the repair: the row panels holding a row
                 // whose second list overflowed are swept again one-sided
                 // (two column halves, lists 0 and 1 of each row written from
                 // scratch), so those rows' lists are exact again
@@ -2783,6 +2857,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                         const int64_t rb = (int64_t)ph[i] * kBM2;
                         MfmaSweepArgs rep = s;
                         rep.sym = 0;
+                        rep.wrap = 0;
                         rep.splits = kRepairSplits;
                         rep.plist = plist + i;
                         rep.npl = 1;
@@ -2814,6 +2889,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                 g_tiles_scored += rtiles;
                 MfmaSweepArgs rep = s;
                 rep.sym = 0;
+                rep.wrap = 0;
                 rep.splits = 2;
                 rep.plist = plist;
                 rep.npl = np;

@@ -909,3 +909,62 @@ def test_selection_distances_are_fp32_sums(nq, P, d, metric):
     kth = torch.topk(D, E, dim=1, largest=False).values[:, -1]
     assert (D.gather(1, got).max(1).values <= kth + 2 * bound.max(1).values).all()
     assert (dist.cpu().diff(dim=1) >= 0).all()
+
+
+@pytest.mark.parametrize("n", [513, 768, 1025, 2049, 4100, 8191, 8193, 9216])
+@pytest.mark.parametrize("dtype,metric,d", [("f16", "ip", 64), ("f32", "l2", 192)])
+def test_symmetric_sweep_around_the_circle(opt, n, dtype, metric, d):
+    """Every tile of the circle once: odd and even panel counts (the pairs half
+    way round an even circle are scored from one side), a last panel of one row,
+    several workgroups a panel (their own rows' survivors through the second
+    lists, with and without the queue: d = 64 is one stage a tile) and second
+    lists forced to overflow (the flagged panels swept again).  The lists are the
+    one-sided sweep's up to ties."""
+    X = torch.from_numpy(gaussian(n, d, n + d, metric == "ip")).cuda()
+    if dtype == "f16":
+        X = X.half()
+    C = 128
+    opt(sweep_sym=0)
+    wi, wd = B.knn_candidates(X, C, metric=metric)
+    nt = (n + 255) // 256
+    for fcap in (0, 40):
+        opt(sweep_sym=1, sweep_sym_fcap=fcap)
+        gi, gd = B.knn_candidates(X, C, metric=metric)
+        from swann_amd import _lib
+        tiles = int(_lib.lib().swann_sweep_tiles_scored())
+        assert tiles == nt * (nt + 1) // 2 if fcap == 0 else tiles > 0
+        assert torch.equal(gd, wd)
+        # equal distances may swap ids; everything else is the same
+        diff = gi != wi
+        if diff.any():
+            tied = torch.zeros_like(diff)
+            tied[:, 1:] |= wd[:, 1:] == wd[:, :-1]
+            tied[:, :-1] |= wd[:, 1:] == wd[:, :-1]
+            tied[:, -1] |= True                    # a tie past the list's end
+            assert (tied | ~diff).all()
+
+
+def test_fp16_sweep_under_graph_capture():
+    """A stream under capture cannot read the symmetric sweep's overflow count
+    back: the sweep is recorded one-sided, and every replay equals the eager
+    one."""
+    X = torch.from_numpy(gaussian(9000, 128, 5, True)).cuda().half()
+    wi, wd = B.knn_candidates(X, 32)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        B.knn_candidates(X, 32)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gi, gd = B.knn_candidates(X, 32)
+    for _ in range(3):
+        gi.zero_()
+        gd.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gd, wd)
+        assert (gi != wi).float().mean() < 1e-5
+        B.knn_candidates(X, 32)
+        torch.cuda.synchronize()
