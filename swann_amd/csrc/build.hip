@@ -23,7 +23,7 @@ namespace swann {
 
 int64_t sweep_mfma_extra_bytes(int64_t n, int dim, int x_dtype);
 int sweep_mfma_cap(int C);
-int sweep_mfma_splits(int64_t n, int dim);
+int sweep_mfma_splits(int64_t n);
 int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, int C, int cap,
                    int splits, float* bkey, int32_t* bid, int32_t* bcnt, char* extra,
                    hipStream_t st, int* used, const int32_t** perm_out);
@@ -296,7 +296,9 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 // 2t + l/32 of its row: fp16 -- 8 halves, one 32x32x16 MFMA; fp32 -- 4
 // floats, four 32x32x2 MFMAs (k = 4*(l/32) + s of the step's 8, a
 // permutation of the K order, which a sum over k does not see).  Products
-// are exact (fp16) or fp32 (fp32), sums fp32.  dim % 8 (fp16: % 16) == 0.
+// are exact (fp16) or fp32 (fp32), sums fp32.  VEC: rows of whole 16-byte chunks
+// on a 16-byte boundary; otherwise element loads, zero past the row's end (as a
+// chunk past it is).
 //
 // PLANES (fp32 rows): each staged float y = x / s_r (s_r a power of two with
 // |y| < 2^15 for the whole row) is split into hi = fp16(y) and lo =
@@ -313,7 +315,7 @@ typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int pswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <typename XT, bool PLANES = false>
+template <typename XT, bool PLANES = false, bool VEC = true>
 __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, const int* cid,
                                  int C, float* gram, float* vn, unsigned char* stg,
                                  const float* srow = nullptr) {
@@ -366,7 +368,18 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
             const int k = k0 + ((q * 256 + tid) & 7) * EPC;
             const bool ok = sid[q] >= 0 && k < dim;
             const int64_t off = ok ? (int64_t)sid[q] * dim + k : 0;
-            dst[q] = *reinterpret_cast<const uint4*>(X + off);
+            if constexpr (VEC) {
+                dst[q] = *reinterpret_cast<const uint4*>(X + off);
+            } else {
+                struct { XT v[EPC]; } part;
+#pragma unroll
+                for (int e = 0; e < EPC; ++e) {
+                    const bool in = ok && k + e < dim;
+                    const XT x = X[in ? off + e : 0];
+                    part.v[e] = in ? x : (XT)0.f;
+                }
+                dst[q] = __builtin_bit_cast(uint4, part);
+            }
             okm |= (ok ? 1u : 0u) << q;
         }
     };
@@ -527,7 +540,7 @@ __global__ __launch_bounds__(256) void row_scale(const float* __restrict__ X, in
 
 // At least two workgroups a CU: the split-plane Gram's fragments and its six
 // accumulator tiles otherwise take 300 registers a wave, one workgroup a CU.
-template <typename XT, bool MFMA, bool PLANES = false>
+template <typename XT, bool MFMA, bool PLANES = false, bool VEC = true>
 __global__ __launch_bounds__(256, 2) void prune_kernel(const XT* __restrict__ X, int64_t n,
                                                     int dim, int metric,
                                                     const int32_t* __restrict__ cand,
@@ -569,7 +582,7 @@ __global__ __launch_bounds__(256, 2) void prune_kernel(const XT* __restrict__ X,
         for (int i = tid; i < C; i += 256)
             if (cid[i] >= 0 && cid[i] < n) atomicMax(&s_nv, i + 1);
         __syncthreads();
-        gram_mfma_staged<XT, PLANES>(X, n, dim, cid, s_nv, gram, vn, stg, srow);
+        gram_mfma_staged<XT, PLANES, VEC>(X, n, dim, cid, s_nv, gram, vn, stg, srow);
     } else {
     // thread (ty, tx) accumulates Gram rows ty*8.., columns tx*8.. (C <= 128)
     float acc[8][8] = {};
@@ -1051,11 +1064,19 @@ int sweep_cap(int C) {
     return cap > 1024 ? 1024 : cap;
 }
 
-bool use_mfma(int dim) { return dim % 8 == 0; }
+// The sweep's tiles run on MFMA at every width, but for fp32 rows that are no
+// multiple of 8 and too wide for the re-rank (their lists come from the SIMT
+// tiles, which need none).
+constexpr int kRerankMax = 16384;
+bool use_mfma(int dim, int x_dtype) {
+    return x_dtype == SWANN_DTYPE_F16 || dim % 8 == 0 || dim <= kRerankMax;
+}
 
 // An fp32 corpus on the MFMA path is swept on an fp16 screen and its lists
 // re-ranked in exact fp32; fp16 corpora and the fp32 SIMT sweep are exact.
-bool screened(int x_dtype, int dim) { return x_dtype == SWANN_DTYPE_F32 && use_mfma(dim); }
+bool screened(int x_dtype, int dim) {
+    return x_dtype == SWANN_DTYPE_F32 && use_mfma(dim, x_dtype);
+}
 
 // Candidates the fp32 screen keeps per row before the exact re-rank (at
 // least C: when C + 32 exceeds n or the sweep's list limit the screen keeps
@@ -1080,11 +1101,11 @@ extern "C" {
 
 int64_t swann_sweep_workspace_size(int64_t n, int dim, int x_dtype, int C) {
     const int Cs = screen_count(C, n, x_dtype, dim);
-    const int cap = use_mfma(dim) ? sweep_mfma_cap(Cs) : sweep_cap(C);
-    const int64_t G = use_mfma(dim) ? sweep_mfma_splits(n, dim) : 1;
+    const int cap = use_mfma(dim, x_dtype) ? sweep_mfma_cap(Cs) : sweep_cap(C);
+    const int64_t G = use_mfma(dim, x_dtype) ? sweep_mfma_splits(n) : 1;
     int64_t b = align256(n * 4) + align256(n * G * cap * 4) * 2 + align256(n * G * 4);
     if (screened(x_dtype, dim)) b += align256(n * (int64_t)Cs * 4) * 2;
-    if (use_mfma(dim)) b += sweep_mfma_extra_bytes(n, dim, x_dtype);
+    if (use_mfma(dim, x_dtype)) b += sweep_mfma_extra_bytes(n, dim, x_dtype);
     return b;
 }
 
@@ -1101,12 +1122,12 @@ int swann_build_sweep(const void* X, int x_dtype, int64_t n, int dim, int metric
     SWANN_REQUIRE(n <= INT32_MAX / 2, "sweep: n too large");
     SWANN_REQUIRE(X && cand && cdist && workspace, "sweep: a required pointer is NULL");
     hipStream_t st = (hipStream_t)stream;
-    const bool mf = use_mfma(dim);
+    const bool mf = use_mfma(dim, x_dtype);
     const int Cs = screen_count(C, n, x_dtype, dim);
     const bool rerank = screened(x_dtype, dim);
-    SWANN_REQUIRE(!rerank || dim * 4 <= 64 * 1024, "sweep: dimension too large for the re-rank");
+    SWANN_REQUIRE(!rerank || dim <= kRerankMax, "sweep: dimension too large for the re-rank");
     const int cap = mf ? sweep_mfma_cap(Cs) : sweep_cap(C);
-    const int G = mf ? sweep_mfma_splits(n, dim) : 1;
+    const int G = mf ? sweep_mfma_splits(n) : 1;
     char* ws = (char*)workspace;
     float* xn = (float*)ws; ws += align256(n * 4);
     float* bkey = (float*)ws; ws += align256(n * (int64_t)G * cap * 4);
@@ -1185,36 +1206,31 @@ int prune_run(const void* X, int x_dtype, int64_t n, int dim, int metric, const 
               const float* cdist, int C, int deg, float alpha, const int32_t* deg_per_node,
               const uint8_t* protect, int32_t* out, const int32_t* order, float* rscale,
               hipStream_t st) {
-    // the Gram on MFMA: fp16 rows with 16-byte aligned 16-wide K steps, fp32
-    // rows with 16-byte aligned 8-wide K steps
+    // the Gram on MFMA (option prune_simt: on SIMT): 16-byte loads where the
+    // rows are whole aligned chunks, element loads otherwise (20,011 rows of 100
+    // fp32, C = 64: 1.04 ms, on SIMT 1.35)
     const bool simt = option_on(kOptPruneSimt);
-    const bool mfma16 = x_dtype == SWANN_DTYPE_F16 && dim % 16 == 0 && (uintptr_t)X % 16 == 0;
-    const bool mfma32 = x_dtype == SWANN_DTYPE_F32 && dim % 8 == 0 && (uintptr_t)X % 16 == 0;
+    const bool f32 = x_dtype == SWANN_DTYPE_F32;
+    const bool vec = dim % (f32 ? 4 : 8) == 0 && (uintptr_t)X % 16 == 0;
     // fp32 rows with a workspace for their scales: the Gram on split fp16
     // planes (option prune_f32 keeps the fp32 MFMA Gram)
-    const bool planes = mfma32 && rscale && !option_on(kOptPruneF32);
-    if (!simt && mfma16)
-        hipLaunchKernelGGL((prune_kernel<_Float16, true>), dim3((unsigned)n), dim3(256), 0, st,
-                           (const _Float16*)X, n, dim, metric, cand, cdist, C, deg, alpha,
-                           deg_per_node, protect, out, nullptr, order);
-    else if (!simt && planes) {
-        hipLaunchKernelGGL(row_scale, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st,
-                           (const float*)X, n, dim, rscale);
-        hipLaunchKernelGGL((prune_kernel<float, true, true>), dim3((unsigned)n), dim3(256), 0,
-                           st, (const float*)X, n, dim, metric, cand, cdist, C, deg, alpha,
-                           deg_per_node, protect, out, rscale, order);
-    } else if (!simt && mfma32)
-        hipLaunchKernelGGL((prune_kernel<float, true>), dim3((unsigned)n), dim3(256), 0, st,
-                           (const float*)X, n, dim, metric, cand, cdist, C, deg, alpha,
-                           deg_per_node, protect, out, nullptr, order);
-    else
-        SWANN_BY_DTYPE(x_dtype,
-            hipLaunchKernelGGL((prune_kernel<float, false>), dim3((unsigned)n), dim3(256), 0, st,
-                               (const float*)X, n, dim, metric, cand, cdist, C, deg, alpha,
-                               deg_per_node, protect, out, nullptr, order),
-            hipLaunchKernelGGL((prune_kernel<_Float16, false>), dim3((unsigned)n), dim3(256), 0,
-                               st, (const _Float16*)X, n, dim, metric, cand, cdist, C, deg, alpha,
-                               deg_per_node, protect, out, nullptr, order));
+    const bool planes = f32 && vec && dim % 8 == 0 && rscale && !option_on(kOptPruneF32);
+    auto launch = [&](auto* kernel, auto* rows, const float* scales) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(256), 0, st, rows, n, dim, metric, cand,
+                           cdist, C, deg, alpha, deg_per_node, protect, out, scales, order);
+    };
+    const float* xf = (const float*)X;
+    const _Float16* xh = (const _Float16*)X;
+    if (simt && f32) launch(prune_kernel<float, false>, xf, nullptr);
+    else if (simt) launch(prune_kernel<_Float16, false>, xh, nullptr);
+    else if (planes) {
+        hipLaunchKernelGGL(row_scale, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, xf, n, dim,
+                           rscale);
+        launch(prune_kernel<float, true, true>, xf, rscale);
+    } else if (f32 && vec) launch(prune_kernel<float, true>, xf, nullptr);
+    else if (f32) launch(prune_kernel<float, true, false, false>, xf, nullptr);
+    else if (vec) launch(prune_kernel<_Float16, true>, xh, nullptr);
+    else launch(prune_kernel<_Float16, true, false, false>, xh, nullptr);
     return launch_status("prune");
 }
 }  // namespace

@@ -59,10 +59,10 @@ __device__ __forceinline__ float dist_formula(float dot, float na, float nb) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 rows -> (hi, lo, scale); fp16 rows -> norms only.
+// fp32 rows -> (hi, scale); fp16 rows -> norms only.
+// Rows of the plane are `ld` wide, zero past the corpus's dim.
 __global__ __launch_bounds__(256) void split_rows(const float* __restrict__ X, int64_t n, int dim,
-                                                  _Float16* __restrict__ hi,
-                                                  _Float16* __restrict__ lo,
+                                                  int ld, _Float16* __restrict__ hi,
                                                   float* __restrict__ scale,
                                                   float* __restrict__ norm) {
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -85,13 +85,58 @@ __global__ __launch_bounds__(256) void split_rows(const float* __restrict__ X, i
     if (m > 0.f) { frexpf(m, &e); }
     const float s = ldexpf(1.0f, e);
     const float inv = ldexpf(1.0f, -e);
+    for (int t = lane; t < ld; t += 64) hi[r * ld + t] = t < dim ? (_Float16)(x[t] * inv) : (_Float16)0.f;
+    if (lane == 0) { scale[r] = s; norm[r] = s2; }
+}
+
+// fp32 rows of a width that is no multiple of 8, as two planes whose product is
+// the fp32 product to about 2^-22 of each factor: y = x / s (s a power of two,
+// |y| < 2^15) is hi = fp16(y) plus lo = fp16(y - hi), and the row panel's rows
+// [hi hi lo] against the column panel's [hi lo hi] give hi.hi + hi.lo + lo.hi.
+// k8 halves a part, the rows `ld` wide with zeros past the parts.
+__global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, int64_t n, int dim,
+                                                   int k8, int ld, _Float16* __restrict__ pa,
+                                                   _Float16* __restrict__ pb,
+                                                   float* __restrict__ scale,
+                                                   float* __restrict__ norm) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (r >= n) return;
+    const float* x = X + r * dim;
+    float m = 0.f, s2 = 0.f;
     for (int t = lane; t < dim; t += 64) {
-        const float v = x[t] * inv;
-        const _Float16 h = (_Float16)v;
-        hi[r * dim + t] = h;
-        if (lo) lo[r * dim + t] = (_Float16)((v - (float)h) * 2048.0f);
+        const float v = x[t];
+        m = fmaxf(m, fabsf(v));
+        s2 = __builtin_fmaf(v, v, s2);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, off, 64));
+        s2 += __shfl_xor(s2, off, 64);
+    }
+    int e = 15;
+    if (m > 0.f && m <= FLT_MAX) frexpf(m, &e);        // m < 2^e
+    e = e - 15 < -126 ? -111 : e;
+    const float s = ldexpf(1.0f, e - 15);
+    const float inv = 1.0f / s;
+    for (int t = lane; t < ld; t += 64) {
+        const int part = t / k8, k = t - part * k8;
+        const float y = part < 3 && k < dim ? x[k] * inv : 0.f;
+        const _Float16 h = (_Float16)y;
+        const _Float16 l = (_Float16)(y - (float)h);
+        pa[r * ld + t] = part == 2 ? l : h;
+        pb[r * ld + t] = part == 1 ? l : h;
     }
     if (lane == 0) { scale[r] = s; norm[r] = s2; }
+}
+
+// fp16 rows copied to a plane `ld` wide, zero past dim.
+__global__ __launch_bounds__(256) void pad_rows(const _Float16* __restrict__ X, int64_t n, int dim,
+                                                int ld, _Float16* __restrict__ out) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= n) return;
+    for (int t = threadIdx.x & 63; t < ld; t += 64)
+        out[r * ld + t] = t < dim ? X[r * dim + t] : (_Float16)0.f;
 }
 
 // The spread of an fp32 corpus's row maxima: rng[0] the largest and rng[1] the
@@ -151,7 +196,7 @@ __global__ void range_init(int* rng) {
 // unscaled kernel (no per-score scale products).  Norms as split_rows
 // computes them (the same order), so the re-rank's are unchanged.
 __global__ __launch_bounds__(256) void rows_to_f16(const float* __restrict__ X, int64_t n, int dim,
-                                                   _Float16* __restrict__ hi,
+                                                   int ld, _Float16* __restrict__ hi,
                                                    float* __restrict__ norm) {
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -161,8 +206,9 @@ __global__ __launch_bounds__(256) void rows_to_f16(const float* __restrict__ X, 
     for (int t = lane; t < dim; t += 64) {
         const float v = x[t];
         s2 = __builtin_fmaf(v, v, s2);
-        hi[r * dim + t] = (_Float16)v;
+        hi[r * ld + t] = (_Float16)v;
     }
+    for (int t = dim + lane; t < ld; t += 64) hi[r * ld + t] = (_Float16)0.f;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s2 += __shfl_xor(s2, off, 64);
     if (lane == 0) norm[r] = s2;
@@ -183,8 +229,10 @@ __global__ __launch_bounds__(256) void norms_f16(const _Float16* __restrict__ X,
 
 // ---------------------------------------------------------------------------
 struct MfmaSweepArgs {
-    const _Float16* hi; const _Float16* lo; const float* scale; const float* xn;
-    int64_t n; int dim; int metric; int C; int cap;
+    // the plane's rows, and where the two sides differ (split3_rows) the column
+    // panels' (else hi again)
+    const _Float16* hi; const _Float16* cols; const float* scale; const float* xn;
+    int64_t n; int dim; int metric; int C; int cap;      // dim: the plane's width
     float* bkey; int32_t* bid; int32_t* bcnt;
     int scaled;                  // rows carry a power-of-two scale (fp32 corpus)
     int splits;                  // column splits G: row r's buffer s is (r * G + s) * cap
@@ -909,7 +957,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
         const int buf = t & 1;
         const int k0 = kt * kBK3;
         const _Float16* ba = X + (int64_t)r0 * dim + k0;
-        const _Float16* bb = X + (int64_t)cb * dim + k0;
+        const _Float16* bb = a.cols + (int64_t)cb * dim + k0;
         // The lane offsets are recomputed at every issue (a few VALU) rather
         // than held across the loop: held, they are the first registers the
         // allocator spills, and each reload's wait (vmcnt counts scratch
@@ -2258,6 +2306,20 @@ __global__ __launch_bounds__(256) void repair_merge(const float* __restrict__ rk
 
 inline int64_t al256(int64_t b) { return ((b + 255) / 256) * 256; }
 
+// The plane the tiles are read from: rows of whole K stages (64 halves).  An fp16
+// corpus of such a width is its own plane; another width is copied, zero past
+// the row's end.  An fp32 corpus is rounded to fp16 (a screen), except at widths
+// that are no multiple of 8, where the sweep has always ranked in fp32: those
+// take three parts a row (split3_rows), so their lists are chosen to fp32
+// accuracy still.
+inline bool plane_split3(int dim, int x_dtype) {
+    return x_dtype == SWANN_DTYPE_F32 && dim % 8 != 0;
+}
+inline int plane_width(int dim, int x_dtype) {
+    const int k = plane_split3(dim, x_dtype) ? 3 * ((dim + 7) / 8 * 8) : dim;
+    return (k + kBK3 - 1) / kBK3 * kBK3;
+}
+
 inline int64_t prune_bytes(int64_t n, int dim);
 
 inline int64_t seed_bytes(int64_t n, int dim) {
@@ -2356,30 +2418,49 @@ inline int sweep_waves() { return option(kOptSweepWaves) == 8 ? 8 : 16; }
 // The buffers hold `splits` lists of `cap` per row (sweep_mfma_splits); *used
 // returns how many the launched kernel filled (the register-staged kernel
 // fills one), which is what the merge must read.
-int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, int C, int cap,
+int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, int C, int cap,
                    int splits, float* bkey, int32_t* bid, int32_t* bcnt, char* extra,
                    hipStream_t st, int* used, const int32_t** perm_out) {
     *perm_out = nullptr;
+    const int dim = plane_width(xdim, x_dtype);          // from here on, the plane's
+    const bool split3 = plane_split3(xdim, x_dtype);
     g_tiles_scored = 0;
     g_dense_panels = 0;
     const int64_t ntile_all = (n + kBM2 - 1) / kBM2;
     float* xn = (float*)extra; extra += al256(n * 4);
     float* scale = (float*)extra; extra += al256(n * 4);
     const _Float16* hi;
+    const _Float16* cols = nullptr;      // the column panels' plane, where it is another
     int scaled = x_dtype == SWANN_DTYPE_F16 ? 0 : 1;
     const unsigned nrb = (unsigned)((n + 3) / 4);
     if (!scaled) {
         hi = (const _Float16*)X;
-        hipLaunchKernelGGL(norms_f16, dim3(nrb), dim3(256), 0, st, hi, n, dim, xn, scale);
+        hipLaunchKernelGGL(norms_f16, dim3(nrb), dim3(256), 0, st, hi, n, xdim, xn, scale);
+        if (dim != xdim) {
+            _Float16* h = (_Float16*)extra;
+            extra += al256(n * (int64_t)dim * 2);
+            hipLaunchKernelGGL(pad_rows, dim3(nrb), dim3(256), 0, st, (const _Float16*)X, n, xdim,
+                               dim, h);
+            hi = h;
+        }
+    } else if (split3) {
+        _Float16* h = (_Float16*)extra;
+        extra += al256(n * (int64_t)dim * 2);
+        _Float16* hc = (_Float16*)extra;
+        extra += al256(n * (int64_t)dim * 2);
+        hipLaunchKernelGGL(split3_rows, dim3(nrb), dim3(256), 0, st, (const float*)X, n, xdim,
+                           (xdim + 7) / 8 * 8, dim, h, hc, scale, xn);
+        hi = h;
+        cols = hc;
     } else {
         _Float16* h = (_Float16*)extra;
         extra += al256(n * (int64_t)dim * 2);
         // the row maxima's range (in `scale`, unused until split_rows writes it)
         int* rng = (int*)scale;
         hipLaunchKernelGGL(range_init, dim3(1), dim3(64), 0, st, rng);
-        const int vec4 = dim % 4 == 0 && (uintptr_t)X % 16 == 0;
+        const int vec4 = xdim % 4 == 0 && (uintptr_t)X % 16 == 0;
         const unsigned nrr = (unsigned)(nrb < (unsigned)kRangeBlocks ? nrb : kRangeBlocks);
-        hipLaunchKernelGGL(row_range, dim3(nrr), dim3(256), 0, st, (const float*)X, n, dim, vec4,
+        hipLaunchKernelGGL(row_range, dim3(nrr), dim3(256), 0, st, (const float*)X, n, xdim, vec4,
                            rng);
         int hr[2] = {0, 0};
         if (hipMemcpyAsync(hr, rng, sizeof(hr), hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -2389,23 +2470,23 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
         }
         const float gmax = __builtin_bit_cast(float, hr[0]), gmin = __builtin_bit_cast(float, hr[1]);
         if (gmax <= 16384.f && gmin >= 0.0625f && !option_on(kOptSweepRowscale)) {
-            hipLaunchKernelGGL(rows_to_f16, dim3(nrb), dim3(256), 0, st, (const float*)X, n, dim,
-                               h, xn);
+            hipLaunchKernelGGL(rows_to_f16, dim3(nrb), dim3(256), 0, st, (const float*)X, n, xdim,
+                               dim, h, xn);
             scaled = 0;
         } else {
-            hipLaunchKernelGGL(split_rows, dim3(nrb), dim3(256), 0, st, (const float*)X, n, dim,
-                               h, (_Float16*)nullptr, scale, xn);
+            hipLaunchKernelGGL(split_rows, dim3(nrb), dim3(256), 0, st, (const float*)X, n, xdim,
+                               dim, h, scale, xn);
         }
         hi = h;
     }
-    MfmaSweepArgs a{hi, nullptr, scale, xn, n, dim, metric, C, cap, bkey, bid, bcnt, scaled, 1,
+    MfmaSweepArgs a{hi, cols ? cols : hi, scale, xn, n, dim, metric, C, cap, bkey, bid, bcnt, scaled, 1,
                     0, 0, 0, nullptr, nullptr, cap};                 // the rest 0
     const unsigned grid = (unsigned)((n + kBM2 - 1) / kBM2);
     const bool ip = metric == SWANN_METRIC_IP;
     *used = 1;
     // the direct loads address a stage's 256 rows with 32-bit byte offsets
     const bool off32 = (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32);
-    if (dim % kBK3 == 0 && (uintptr_t)hi % 16 == 0 && off32 && !option_on(kOptSweepRegstage)) {
+    if ((uintptr_t)hi % 16 == 0 && off32 && (split3 || !option_on(kOptSweepRegstage))) {
         const int64_t ntile = (n + kBM2 - 1) / kBM2;
         if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !capturing(st)) {
             // symmetric sweep: tile (I, J), J >= I, scored once for the rows of
@@ -2504,7 +2585,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
             int32_t* rid = nullptr;
             int32_t* rcnt = nullptr;
             const int32_t* ordered = nullptr;
-            if (ntile > 2 * kSeedBand && !option_on(kOptSweepNoseed)) {
+            if (ntile > 2 * kSeedBand && !split3 && !option_on(kOptSweepNoseed)) {
                 bool clustered = false;
                 // the order's workspace (seed_bytes, repair_bytes)
                 float* sk = (float*)extra; extra += al256(n * kSketch * 4);
@@ -2529,10 +2610,10 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                 const int P = (int)(pw < 1 ? 1 : pw > kMaxPivots ? kMaxPivots : pw);
                 if (x_dtype == SWANN_DTYPE_F16)
                     hipLaunchKernelGGL(row_sketch<_Float16>, dim3(nrb), dim3(256), 0, st,
-                                       (const _Float16*)X, n, dim, sk);
+                                       (const _Float16*)X, n, xdim, sk);
                 else
                     hipLaunchKernelGGL(row_sketch<float>, dim3(nrb), dim3(256), 0, st,
-                                       (const float*)X, n, dim, sk);
+                                       (const float*)X, n, xdim, sk);
                 hipLaunchKernelGGL(pivot_init, dim3(P), dim3(kSketch), 0, st, sk, n, P, psk);
                 // two k-means steps on the sketches, then the final grouping;
                 // after the first assignment, rows that do not cluster (mean
@@ -2628,6 +2709,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
                     hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
                 MfmaSweepArgs pre = s;
                 pre.hi = hp;
+                pre.cols = hp;
                 pre.xn = xnp;
                 pre.scale = scp;
                 int rc = launch_status("sweep (mfma, seed order)");
@@ -2943,10 +3025,13 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int dim, int metric, i
     return launch_status("sweep (mfma)");
 }
 
-// Extra workspace: norms, scales, (fp32 corpus) the fp16 plane, the
+// Extra workspace: norms, scales, the fp16 plane (an fp32
+// corpus, or an fp16 one of another width than the plane's), the
 // symmetric sweep's thresholds and overflow count, and its seed pre-pass.
-int64_t sweep_mfma_extra_bytes(int64_t n, int dim, int x_dtype) {
-    const int64_t planes = x_dtype == SWANN_DTYPE_F16 ? 0 : 1;
+int64_t sweep_mfma_extra_bytes(int64_t n, int xdim, int x_dtype) {
+    const int dim = plane_width(xdim, x_dtype);
+    const int64_t planes = plane_split3(xdim, x_dtype) ? 2
+                           : x_dtype == SWANN_DTYPE_F16 && dim == xdim ? 0 : 1;
     const int64_t base = al256(n * 4) * 2 + planes * al256(n * (int64_t)dim * 2) +
                          al256(n * 4) + 256 + al256(n * 4);
     // the locality order, seeds and panel repair run only in the symmetric
@@ -2955,7 +3040,7 @@ int64_t sweep_mfma_extra_bytes(int64_t n, int dim, int x_dtype) {
     // run never finds less than it needs: a corpus the clustering check
     // declines at run time, or option sweep_noseed, still reserves it)
     const int64_t ntile = (n + kBM2 - 1) / kBM2;
-    const bool seeded = dim % kBK3 == 0 && sweep_sym(ntile) && ntile > 2 * kSeedBand;
+    const bool seeded = !plane_split3(xdim, x_dtype) && sweep_sym(ntile) && ntile > 2 * kSeedBand;
     return base + (seeded ? seed_bytes(n, dim) + repair_bytes(1024) : 0);   // cap <= 1024
 }
 
@@ -2965,8 +3050,7 @@ int64_t sweep_mfma_extra_bytes(int64_t n, int dim, int x_dtype) {
 #ifndef SWANN_SWEEP_MIN_SPLITS
 #define SWANN_SWEEP_MIN_SPLITS 2
 #endif
-int sweep_mfma_splits(int64_t n, int dim) {
-    if (dim % kBK3 != 0) return 1;
+int sweep_mfma_splits(int64_t n) {
     const int64_t ntile = (n + kBM2 - 1) / kBM2;
     int g = SWANN_SWEEP_MIN_SPLITS;
     while (g < 8 && ntile * g < 512) g *= 2;

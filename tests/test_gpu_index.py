@@ -968,3 +968,36 @@ def test_fp16_sweep_under_graph_capture():
         assert (gi != wi).float().mean() < 1e-5
         B.knn_candidates(X, 32)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("n,d,dtype,C", [(300, 1, "f32", 20), (1000, 7, "f32", 64),
+                                         (2100, 25, "f16", 100), (8500, 100, "f32", 64),
+                                         (2100, 201, "f16", 128), (2100, 200, "f16", 96),
+                                         (2100, 999, "f32", 256), (2100, 72, "f32", 96)])
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+def test_sweep_and_prune_at_any_width(n, d, dtype, C, metric):
+    """Widths that are no whole K stage of the tiles (the corpus copied to a padded
+    plane, or split in three parts where fp32 rows are no multiple of 8) and rows
+    off a 16-byte boundary (the prune's element loads): distances within fp32
+    rounding of the float64 top-C, the prune's rows the SIMT Gram's."""
+    from swann_amd import _lib
+    X = torch.from_numpy(gaussian(n, d, n + d, metric == "ip")).cuda()
+    if dtype == "f16":
+        X = X.half()
+    i, dist = B.knn_candidates(X, C, metric=metric)
+    x = X.double()
+    sq = (x * x).sum(1)
+    D = 1 - x @ x.T if metric == "ip" else (sq[:, None] + sq[None] - 2 * x @ x.T).clamp(min=0)
+    D.fill_diagonal_(float("inf"))
+    want = torch.topk(D, C, dim=1, largest=False).values
+    # d products and sums, then the formula, each within u of their magnitude
+    mag = 1.0 + float((sq if metric == "l2" else x.norm(dim=1) ** 2).max())
+    bound = (2 * d + 8) * 2.0 ** -24 * mag * 2
+    assert (dist.double() - want).abs().max() <= bound
+    assert (D.gather(1, i.long()) - dist.double()).abs().max() <= bound
+    if C <= 128:
+        G = B.robust_prune(X, i, dist, min(C, 48), metric=metric)
+        with _lib.options(prune_simt=1):
+            S_ = B.robust_prune(X, i, dist, min(C, 48), metric=metric)
+        # sums in another order turn a near-tie of the rule in a few rows
+        assert (G != S_).any(1).float().mean() <= 0.005
