@@ -288,11 +288,13 @@ typedef float f32x16v __attribute__((ext_vector_type(16)));
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-// The Gram with the candidate rows staged through LDS, 128 bytes of each
-// row at a time (64 halves or 32 floats), so every row is read from memory
-// once per node instead of once per wave that needs it.  Each 16-byte chunk c
+// The Gram with the candidate rows staged through LDS, 256 bytes of each
+// row at a time (128 halves or 64 floats), so every row is read from memory
+// once per node instead of once per wave that needs it.  What bounds it is that
+// gather: 128 rows of random lines a node, 6.0 TB/s of them at 100,000 x 1,536
+// fp16 (plain gathers of such rows reach 6.3 to 6.6).  Each 16-byte chunk c
 // of row r sits at chunk c ^ swz(r) (the 32 rows of a fragment read fall in
-// distinct banks).  A K chunk is four steps; in step t lane l reads chunk
+// distinct banks).  A K chunk is eight steps; in step t lane l reads chunk
 // 2t + l/32 of its row: fp16 -- 8 halves, one 32x32x16 MFMA; fp32 -- 4
 // floats, four 32x32x2 MFMAs (k = 4*(l/32) + s of the step's 8, a
 // permutation of the K order, which a sum over k does not see).  Products
@@ -302,18 +304,20 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 //
 // PLANES (fp32 rows): each staged float y = x / s_r (s_r a power of two with
 // |y| < 2^15 for the whole row) is split into hi = fp16(y) and lo =
-// fp16(y - hi) (y - hi is exact in fp32), hi in logical chunks 0-3 of the
-// row's 128 bytes, lo in 4-7; the Gram entry is s_a s_b (hi.hi + hi.lo +
+// fp16(y - hi) (y - hi is exact in fp32), hi in logical chunks 0-7 of the
+// row's 256 bytes, lo in 8-15; the Gram entry is s_a s_b (hi.hi + hi.lo +
 // lo.hi), three 32x32x16 f16 MFMAs per 16 of K into one fp32 accumulator
 // (exact products, fp32 sums) for what the fp32 path does in eight 32x32x2
 // f32 MFMAs.  y keeps 22 of its 24 significant bits (the lo.lo term and lo's
 // own rounding are below 2^-22 of the element; lo is subnormal only for
 // elements below 2^-17 of the row's largest), so the Gram differs from the
 // fp32 one by a few of its last bits, like a different summation order.
-constexpr int kStgRow = 128;                       // bytes of a row per K chunk
+constexpr int kStgRow = 256;                       // bytes of a row per K chunk
+constexpr int kStgCh = kStgRow / 16;               // 16-byte pieces of it
+constexpr int kStgPer = kPruneMaxC * kStgCh / 256; // pieces a thread stages
 typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ int pswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+__device__ __forceinline__ int pswz(int r) { return r & (kStgCh - 1); }
 
 template <typename XT, bool PLANES = false, bool VEC = true>
 __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, const int* cid,
@@ -345,27 +349,27 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[x][e] = 0.f;
     const int half = lane >> 5;
-    // staging: 128 rows x 8 chunks, 4 per thread; two K chunks' loads are in
-    // flight ahead of the chunk being multiplied (the kernel waits on memory
-    // latency, not on its MFMAs).  The loads are unconditional -- a lane past
+    // staging: 128 rows x 16 chunks, 8 per thread, whose loads are in flight
+    // while the chunk before is multiplied (the kernel waits on memory latency,
+    // not on its MFMAs).  The loads are unconditional -- a lane past
     // the candidates or the row reads element 0 of the corpus and its bit in
     // the chunk's mask zeroes it at staging -- so that the compiler counts
     // them exactly and each staging waits only for its own chunk.
     const int rows = (C + 31) & ~31;               // rows some tile reads
-    int sid[4];
+    int sid[kStgPer];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int r = (q * 256 + tid) >> 3;
+    for (int q = 0; q < kStgPer; ++q) {
+        const int r = (q * 256 + tid) / kStgCh;
         const int id = r < C ? cid[r] : -1;
         sid[q] = r < rows && id >= 0 && id < n ? id : -1;
     }
-    uint4 nxa[4], nxb[4];
-    unsigned oka = 0u, okb = 0u;
+    uint4 nx[kStgPer];
+    unsigned oka = 0u;
     auto fetch = [&](uint4* dst, unsigned& okm, int k0) {
         okm = 0u;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = k0 + ((q * 256 + tid) & 7) * EPC;
+        for (int q = 0; q < kStgPer; ++q) {
+            const int k = k0 + (tid & (kStgCh - 1)) * EPC;
             const bool ok = sid[q] >= 0 && k < dim;
             const int64_t off = ok ? (int64_t)sid[q] * dim + k : 0;
             if constexpr (VEC) {
@@ -383,16 +387,16 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
             okm |= (ok ? 1u : 0u) << q;
         }
     };
-    // thread t stages rows (q 256 + t) / 8 < 128 of every chunk (all of the
+    // thread t stages rows (q 256 + t) / kStgCh < 128 of every chunk (all of the
     // buffer; rows past the candidates stage zeros), with its rows' scales
-    float inv[4];
+    float inv[kStgPer];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) inv[q] = PLANES ? 1.f / srow[(q * 256 + tid) >> 3] : 1.f;
+    for (int q = 0; q < kStgPer; ++q) inv[q] = PLANES ? 1.f / srow[(q * 256 + tid) / kStgCh] : 1.f;
     auto stage = [&](const uint4* src, unsigned okm) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < kStgPer; ++q) {
             const int e = q * 256 + tid;
-            const int r = e >> 3, c = e & 7;
+            const int r = e / kStgCh, c = e & (kStgCh - 1);
             const uint4 raw = ((okm >> q) & 1u) ? src[q] : make_uint4(0u, 0u, 0u, 0u);
             if constexpr (PLANES) {
                 // floats 4c..4c+3 of the chunk: their hi halves to byte 8c of
@@ -409,7 +413,7 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
                 unsigned char* row = stg + r * kStgRow + ((c & 1) << 3);
                 *reinterpret_cast<uint2*>(row + (((c >> 1) ^ pswz(r)) << 4)) =
                     __builtin_bit_cast(uint2, hi);
-                *reinterpret_cast<uint2*>(row + (((4 + (c >> 1)) ^ pswz(r)) << 4)) =
+                *reinterpret_cast<uint2*>(row + (((kStgCh / 2 + (c >> 1)) ^ pswz(r)) << 4)) =
                     __builtin_bit_cast(uint2, lo);
             } else {
                 *reinterpret_cast<uint4*>(stg + r * kStgRow + ((c ^ pswz(r)) << 4)) = raw;
@@ -418,11 +422,11 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
     };
     auto multiply = [&]() {
         if (PLANES && busy) {
-            // 32 of K a chunk: two 16-wide steps of hi.hi, hi.lo and lo.hi,
+            // 64 of K a chunk: four 16-wide steps of hi.hi, hi.lo and lo.hi,
             // all into one accumulator
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int chh = 2 * t + half, chl = 4 + 2 * t + half;
+            for (int t = 0; t < kStgCh / 4; ++t) {
+                const int chh = 2 * t + half, chl = kStgCh / 2 + 2 * t + half;
 #pragma unroll
                 for (int x = 0; x < 3; ++x) {
                     if (!on[x]) continue;
@@ -440,10 +444,12 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
                     acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[x], 0, 0, 0);
                     acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[x], 0, 0, 0);
                 }
+                // fragments of one step at a time: hoisted further they spill
+                __builtin_amdgcn_sched_barrier(0);
             }
         } else if (busy) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < kStgCh / 2; ++t) {
                 const int ch = 2 * t + half;
 #pragma unroll
                 for (int x = 0; x < 3; ++x) {
@@ -467,34 +473,18 @@ __device__ void gram_mfma_staged(const XT* __restrict__ X, int64_t n, int dim, c
                                                                           0, 0, 0);
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
     // Every fetch is issued, also past the last chunk (then of chunk 0 again,
-    // which is never staged): with no fetch under a branch, each staging
-    // waits for its own four loads only (vmcnt(4)), not for the next chunk's.
-    // Two chunks a trip and no exit inside it, so that at the top of the loop
-    // the compiler sees buffer a's loads as the older ones on every path; an
-    // odd last chunk runs after the loop.
+    // which is never staged): no fetch is under a branch.
     const int nch = (dim + KC - 1) / KC;
-    fetch(nxa, oka, 0);
-    fetch(nxb, okb, nch > 1 ? KC : 0);
-    int ch = 0;
-    for (; ch + 1 < nch; ch += 2) {
-        stage(nxa, oka);
+    fetch(nx, oka, 0);
+    for (int ch = 0; ch < nch; ++ch) {
+        stage(nx, oka);
         __syncthreads();
-        fetch(nxa, oka, ch + 2 < nch ? (ch + 2) * KC : 0);
-        multiply();
-        __syncthreads();
-        stage(nxb, okb);
-        __syncthreads();
-        fetch(nxb, okb, ch + 3 < nch ? (ch + 3) * KC : 0);
-        multiply();
-        __syncthreads();
-    }
-    if (ch < nch) {
-        stage(nxa, oka);
-        __syncthreads();
+        fetch(nx, oka, ch + 1 < nch ? (ch + 1) * KC : 0);
         multiply();
         __syncthreads();
     }
@@ -538,11 +528,14 @@ __global__ __launch_bounds__(256) void row_scale(const float* __restrict__ X, in
     }
 }
 
-// At least two workgroups a CU: the split-plane Gram's fragments and its six
-// accumulator tiles otherwise take 300 registers a wave, one workgroup a CU.
+// Three workgroups a CU, as many as 168 registers allow (four, at 128, spill:
+// 19.0 ms).  The staged rows and the Gram share their LDS (34 KB a workgroup);
+// apart they took 50 KB.  100,000 nodes of 128 candidates: 7.3 to 6.6 ms (1,536
+// fp16) and 10.9 to 9.9 ms (960 fp32, split planes) against 128-byte chunks two
+// ahead and LDS of its own for each.
 template <typename XT, bool MFMA, bool PLANES = false, bool VEC = true>
-__global__ __launch_bounds__(256, 2) void prune_kernel(const XT* __restrict__ X, int64_t n,
-                                                    int dim, int metric,
+__global__ __launch_bounds__(256, VEC ? 3 : 2) void prune_kernel(const XT* __restrict__ X,
+                                                    int64_t n, int dim, int metric,
                                                     const int32_t* __restrict__ cand,
                                                     const float* __restrict__ cdist, int C,
                                                     int deg, float alpha,
@@ -551,7 +544,10 @@ __global__ __launch_bounds__(256, 2) void prune_kernel(const XT* __restrict__ X,
                                                     int32_t* __restrict__ out,
                                                     const float* __restrict__ rscale = nullptr,
                                                     const int32_t* __restrict__ order = nullptr) {
-    __shared__ float gram[kPruneMaxC * (kPruneMaxC - 1) / 2];
+    // the Gram is written once every staged chunk has been multiplied, so the
+    // staging buffer is its space
+    __shared__ __align__(16) float gram[kPruneMaxC * kPruneMaxC / 2];
+    static_assert(sizeof(gram) >= kPruneMaxC * kStgRow, "the staged rows fit");
     __shared__ float vn[kPruneMaxC];
     __shared__ float Vs[MFMA ? 1 : kPKC][kPruneMaxC + 4];
     __shared__ int cid[kPruneMaxC];
@@ -568,7 +564,7 @@ __global__ __launch_bounds__(256, 2) void prune_kernel(const XT* __restrict__ X,
     __syncthreads();
     if constexpr (MFMA) {
         // candidates past the last valid one are never read: the Gram stops there
-        __shared__ __align__(16) unsigned char stg[kPruneMaxC * kStgRow];
+        unsigned char* stg = reinterpret_cast<unsigned char*>(gram);
         __shared__ float srow[PLANES ? kPruneMaxC : 1];
         __shared__ int s_nv;
         if (tid == 0) s_nv = 0;
