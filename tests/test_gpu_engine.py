@@ -817,3 +817,39 @@ def test_build_codes_at_row_and_word_edges(n, d, dtype):
         words = (bits.view(n, -1, 32) << torch.arange(32)).sum(2)
         assert torch.equal(codes.long() & 0xFFFFFFFF, words)
         assert torch.allclose(alpha, df.double().abs().mean(1).float(), rtol=2.0 ** -23)
+
+
+@pytest.mark.parametrize("team", [4, 8, 16, 32, 64])
+@pytest.mark.parametrize("d,deg,dtype", [(33, 31, "f32"), (64, 64, "f16"), (40, 97, "f16"),
+                                         (96, 128, "f32")])
+def test_eager_claims_equal_the_listed_ones(team, d, deg, dtype):
+    """Sixteen waves a branch with claim bits: a neighbour's row is read together
+    with its claim, and the bound a step ahead.  One branch a launch, several
+    expansions each (the bound is then only the branch's own and the earlier
+    branches'), the state equals the one-wave kernel's bit for bit: queues and
+    every counter."""
+    from swann_amd import _lib
+    n, nq, J, L, budget = 1500, 3, 4, 24, 18
+    g = torch.Generator().manual_seed(d + team)
+    X = torch.randn((n, d), generator=g).cuda()
+    X /= X.norm(dim=1, keepdim=True)
+    X = X.half() if dtype == "f16" else X
+    G = torch.randint(-1, n, (n, deg), generator=g, dtype=torch.int32).cuda()
+    Q = torch.randn((nq, d), generator=g).cuda()
+    Q /= Q.norm(dim=1, keepdim=True)
+    seeds = torch.randint(0, n, (nq, J), generator=g, dtype=torch.int32)
+    states = []
+    for block in (64, 1024):
+        with _lib.options(search_block=block):
+            st = E.init_states(X, Q, seeds, L=L, B=budget, D=deg, team_size=team, stop_eps=0.2,
+                               kstop=10, shared_cache=True, shared_bound=True, exclusive=True,
+                               elide_visited=True, claim_bits=True)
+            for _ in range(budget // 6):
+                for j in range(J):
+                    act = torch.arange(nq, dtype=torch.int32, device=DEV) * J + j
+                    E.advance(X, G, Q, st, 6, active=act)
+        states.append(st)
+    a, b = states
+    for f in ("ids", "dist", "expanded", "lineage", "counters", "cache_id", "bound"):
+        assert torch.equal(getattr(a, f), getattr(b, f)), f
+    assert int(a.counters[..., 4].sum()) > 0
