@@ -70,6 +70,8 @@ __global__ __launch_bounds__(256) void row_norms(const float* __restrict__ A, in
     if (r >= n) return;
     const float* a = A + r * dim;
     float s = 0.f;
+    // eight loads in flight; the sum's order is the loop's
+#pragma unroll 8
     for (int t = lane; t < dim; t += 64) s = __builtin_fmaf(a[t], a[t], s);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
@@ -186,7 +188,18 @@ __global__ __launch_bounds__(256) void dist_gemm(const float* __restrict__ A,
     fetch(kb + kGK);
     __syncthreads();
     int buf = 0;
+    f32x4 fga[2][BI], fgb[2][BI];
+    auto frags = [&](int t, int slot) {
+        const int co = ((2 * t + half) ^ fsw) << 4;
+#pragma unroll
+        for (int i = 0; i < BI; ++i) {
+            const int r = i * 32 + (lane & 31);
+            fga[slot][i] = *reinterpret_cast<const f32x4*>(&sA[buf][(wm + r) * kGRow + co]);
+            fgb[slot][i] = *reinterpret_cast<const f32x4*>(&sB[buf][(wn + r) * kGRow + co]);
+        }
+    };
     for (int k0 = kb; k0 < ke; k0 += kGK) {
+        frags(0, 0);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             // half way, the next stage goes to the other buffer (last read
@@ -197,14 +210,12 @@ __global__ __launch_bounds__(256) void dist_gemm(const float* __restrict__ A,
                 stage(buf ^ 1);
                 fetch(k0 + 2 * kGK);
             }
-            const int co = ((2 * t + half) ^ fsw) << 4;
-            f32x4 fa[BI], fb[BI];
-#pragma unroll
-            for (int i = 0; i < BI; ++i) {
-                const int r = i * 32 + (lane & 31);
-                fa[i] = *reinterpret_cast<const f32x4*>(&sA[buf][(wm + r) * kGRow + co]);
-                fb[i] = *reinterpret_cast<const f32x4*>(&sB[buf][(wn + r) * kGRow + co]);
-            }
+            // the next step's fragments are read while this one's multiply
+            if (t < 3) frags(t + 1, (t + 1) & 1);
+            // (in that order, where four blocks' MFMAs cover the reads)
+            if (BI > 1) __builtin_amdgcn_sched_barrier(0);
+            const f32x4* fa = fga[t & 1];
+            const f32x4* fb = fgb[t & 1];
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
