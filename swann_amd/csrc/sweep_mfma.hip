@@ -94,6 +94,10 @@ __global__ __launch_bounds__(256) void split_rows(const float* __restrict__ X, i
 // |y| < 2^15) is hi = fp16(y) plus lo = fp16(y - hi), and the row panel's rows
 // [hi hi lo] against the column panel's [hi lo hi] give hi.hi + hi.lo + lo.hi.
 // k8 halves a part, the rows `ld` wide with zeros past the parts.
+// An infinite (or NaN) element has no lo and stands in the first part only, where
+// it meets the other row's hi and is infinite with that one's sign, as the fp32
+// product is; so a nonzero y's hi is never zero (at least 2^-24, which lo then
+// takes back), and the row's scale is that of its finite elements.
 __global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, int64_t n, int dim,
                                                    int k8, int ld, _Float16* __restrict__ pa,
                                                    _Float16* __restrict__ pb,
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, 
     float m = 0.f, s2 = 0.f;
     for (int t = lane; t < dim; t += 64) {
         const float v = x[t];
-        m = fmaxf(m, fabsf(v));
+        m = fmaxf(m, fabsf(v) <= FLT_MAX ? fabsf(v) : 0.f);
         s2 = __builtin_fmaf(v, v, s2);
     }
 #pragma unroll
@@ -115,17 +119,20 @@ __global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, 
         s2 += __shfl_xor(s2, off, 64);
     }
     int e = 15;
-    if (m > 0.f && m <= FLT_MAX) frexpf(m, &e);        // m < 2^e
+    if (m > 0.f) frexpf(m, &e);                        // m < 2^e
     e = e - 15 < -126 ? -111 : e;
     const float s = ldexpf(1.0f, e - 15);
     const float inv = 1.0f / s;
     for (int t = lane; t < ld; t += 64) {
         const int part = t / k8, k = t - part * k8;
         const float y = part < 3 && k < dim ? x[k] * inv : 0.f;
-        const _Float16 h = (_Float16)y;
+        const bool fin = fabsf(y) <= FLT_MAX;
+        _Float16 h = (_Float16)y;
+        if (fin && y != 0.f && h == (_Float16)0.f) h = (_Float16)copysignf(0x1p-24f, y);
         const _Float16 l = (_Float16)(y - (float)h);
-        pa[r * ld + t] = part == 2 ? l : h;
-        pb[r * ld + t] = part == 1 ? l : h;
+        const _Float16 z = (_Float16)0.f;
+        pa[r * ld + t] = part == 0 ? h : !fin ? z : part == 2 ? l : h;
+        pb[r * ld + t] = part == 0 ? h : !fin ? z : part == 1 ? l : h;
     }
     if (lane == 0) { scale[r] = s; norm[r] = s2; }
 }

@@ -1001,3 +1001,44 @@ def test_sweep_and_prune_at_any_width(n, d, dtype, C, metric):
             S_ = B.robust_prune(X, i, dist, min(C, 48), metric=metric)
         # sums in another order turn a near-tie of the rule in a few rows
         assert (G != S_).any(1).float().mean() <= 0.005
+
+
+@pytest.mark.parametrize("d", [25, 65, 100, 201])
+@pytest.mark.parametrize("metric", ["ip", "l2"])
+def test_sweep_ranks_infinite_elements_as_fp32_sums_do(d, metric):
+    """Rows with an infinite element, at widths that are no multiple of 8 (the wider
+    ones are swept as three parts a row): under ip such a row's distance to the others is
+    -inf or +inf by sign, so it leads the lists of those it points at and its own
+    list holds rows at -inf; under l2 its norm is infinite and it is in no list.
+    A NaN row is in no list, and the finite rows' other neighbours are unmoved."""
+    n, C = 2100, 64
+    X = torch.from_numpy(gaussian(n, d, d, metric == "ip"))
+    X[5, 3] = X[1000, 0] = float("inf")
+    X[17, d - 1] = float("-inf")
+    X[30, 1] = float("nan")
+    X[40, 3], X[41] = 1e-20, X[41] * 1e30       # a tiny factor of infinity, a large row
+    X[41, 4] = float("inf")
+    odd = torch.tensor([5, 17, 30, 41, 1000])
+    gi, gd = (t.cpu() for t in B.knn_candidates(X.cuda(), C, metric=metric))
+    x = X.double()
+    sq = (x * x).sum(1)
+    D = 1 - x @ x.T if metric == "ip" else (sq[:, None] + sq[None] - 2 * x @ x.T)
+    D = torch.nan_to_num(D, nan=float("inf"), posinf=float("inf"), neginf=float("-inf"))
+    D.fill_diagonal_(float("inf"))
+    fin = torch.ones(n, dtype=torch.bool)
+    fin[odd] = False
+    want = torch.topk(D, C, dim=1, largest=False).values
+    assert torch.equal(torch.isinf(gd[fin]), torch.isinf(want[fin]))
+    if metric == "ip":
+        got = D.gather(1, gi.long().clamp(min=0))
+        assert torch.isinf(want[fin]).any()
+        assert torch.equal(torch.isinf(got[fin]), torch.isinf(want[fin]))
+        for row in (5, 17, 41, 1000):
+            assert (gd[row] == float("-inf")).all() and (got[row] == float("-inf")).all()
+    else:
+        assert not torch.isin(gi[fin], odd.int()).any()
+    # d products and sums and the formula, each within u of their magnitude
+    mag = 1.0 + float((sq if metric == "l2" else sq.sqrt())[fin].max())
+    both = torch.isfinite(want[fin])
+    bound = (2 * d + 8) * 2.0 ** -24 * mag * 2
+    assert (gd[fin].double() - want[fin])[both].abs().max() <= bound
