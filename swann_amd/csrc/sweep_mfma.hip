@@ -435,7 +435,7 @@ __device__ __forceinline__ void append_own(const f32x16& v, int rbase, int64_t r
             if (nterm_scale == 1)
                 dot = s4[q] * sc * (v[e] + (*vx)[e] * (1.0f / 2048.0f));
             else if (nterm_scale == 2)
-                dot = s4[q] * sc * v[e];
+                dot = s4[q] * v[e] * sc;
             else
                 dot = v[e];
             if (!cok) continue;
@@ -469,7 +469,7 @@ __device__ __forceinline__ void epilogue_block(const f32x16& v, int rbase, int64
         if (nterm_scale == 1)
             dot = s4[q] * sc * (v[e] + (*vx)[e] * (1.0f / 2048.0f));
         else if (nterm_scale == 2)
-            dot = s4[q] * sc * v[e];
+            dot = s4[q] * v[e] * sc;
         else
             dot = v[e];
         return dist_formula<METRIC>(dot, METRIC == SWANN_METRIC_L2 ? r4[q] : 0.f, cn);
@@ -492,7 +492,7 @@ __device__ __forceinline__ void epilogue_block(const f32x16& v, int rbase, int64
                                           : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float dot = nterm_scale ? s4[q] * sc * v[g * 4 + q] : v[g * 4 + q];
+                const float dot = nterm_scale ? s4[q] * v[g * 4 + q] * sc : v[g * 4 + q];
                 any = any || (METRIC == SWANN_METRIC_IP ? dot > h4[q] : dot > ch + h4[q]);
             }
         }
@@ -543,7 +543,7 @@ __device__ __forceinline__ void queue_foreign(const f32x16& v, int rbase, int64_
                               : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float dot = scaled ? s4[q] * sc * v[g * 4 + q] : v[g * 4 + q];
+            const float dot = scaled ? s4[q] * v[g * 4 + q] * sc : v[g * 4 + q];
             if (!cok) continue;
             const float d = dist_formula<METRIC>(dot, cn, r4[q]);
             const int rl = rbase + g * 8 + q;
@@ -588,14 +588,14 @@ __device__ __forceinline__ void screen_pair(const f32x16& v, int rbase, float cn
                                   : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float dot = SCALED ? s4[q] * sc * v[g * 4 + q] : v[g * 4 + q];
+                const float dot = SCALED ? s4[q] * v[g * 4 + q] * sc : v[g * 4 + q];
                 o |= __ballot(METRIC == SWANN_METRIC_L2 ? dot > ch + t4[q] : dot > t4[q]);
                 f |= __ballot(METRIC == SWANN_METRIC_L2 ? dot > h + f4[q] : dot > h);
             }
         } else {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float dot = SCALED ? s4[q] * sc * v[g * 4 + q] : v[g * 4 + q];
+                const float dot = SCALED ? s4[q] * v[g * 4 + q] * sc : v[g * 4 + q];
                 o |= __ballot(METRIC == SWANN_METRIC_L2 ? dot > ch + t4[q] : dot > t4[q]);
             }
         }
@@ -910,11 +910,15 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
     const int r0 = (a.sym ? lid : a.plist ? a.plist[lid / G] : lid / G) * kBM2;
     const int split = a.sym ? 0 : lid % G;
 
+    // a score is (row scale * sum) * column scale; the three parts' sums reach
+    // 2^30 a product, which the row's scale takes back first, so that nothing
+    // overflows or underflows on the way to a distance that does not
+    const float sdn = a.hi != a.cols ? 0x1p-15f : 1.f;
     if (tid < kBM2) {
         thr[tid] = r0 + tid >= n ? -INFINITY : a.sym ? a.gthr[r0 + tid] : INFINITY;
         cnt[tid] = (a.sym && r0 + tid < n) ? a.bcnt[(int64_t)(r0 + tid) * 2] : 0;
         rnorm[tid] = (r0 + tid < n) ? a.xn[r0 + tid] : 0.f;
-        if (SCALED) rscale[tid] = (r0 + tid < n) ? a.scale[r0 + tid] : 1.f;
+        if (SCALED) rscale[tid] = (r0 + tid < n) ? a.scale[r0 + tid] * sdn : 1.f;
         sthr[tid] = screen_thr<METRIC>(thr[tid], rnorm[tid]);
         if (METRIC == SWANN_METRIC_L2) frow[tid] = 0.5f * (rnorm[tid] - 1e-5f * fabsf(rnorm[tid]));
     }
@@ -1053,7 +1057,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
             for (int j = 0; j < BJ; ++j) {
                 const int c = cbt + wn * CW + j * 32 + (lane & 31);
                 if (METRIC == SWANN_METRIC_L2) cn[j] = c < n ? a.xn[c] : 0.f;
-                if (SCALED) cs[j] = c < n ? a.scale[c] : 1.f;
+                if (SCALED) cs[j] = c < n ? a.scale[c] * (a.hi != a.cols ? 0x1p15f : 1.f) : 1.f;
             }
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0): this wave's stage-t loads

@@ -1042,3 +1042,17 @@ def test_sweep_ranks_infinite_elements_as_fp32_sums_do(d, metric):
     both = torch.isfinite(want[fin])
     bound = (2 * d + 8) * 2.0 ** -24 * mag * 2
     assert (gd[fin].double() - want[fin])[both].abs().max() <= bound
+
+
+@pytest.mark.parametrize("power", [-61, 40])
+@pytest.mark.parametrize("d", [100, 104])
+def test_sweep_lists_do_not_depend_on_the_rows_scale(d, power):
+    """Rows times a power of two that leaves every l2 distance a normal number
+    (2^-61: about 2^-115) give the same lists, the distances times its square, both
+    on the three-part planes (d = 100) and on the scaled screen (d = 104)."""
+    X = torch.from_numpy(gaussian(2100, d, d, False)).cuda()
+    wi, wd = B.knn_candidates(X, 64, metric="l2")
+    gi, gd = B.knn_candidates(X * 2.0 ** power, 64, metric="l2")
+    # products below the normal range lose bits, so a distance may move by an ulp
+    assert torch.allclose(gd * 2.0 ** -power * 2.0 ** -power, wd, rtol=1e-6, atol=0)
+    assert (gi != wi).float().mean() < 1e-3
