@@ -1060,12 +1060,18 @@ int sweep_cap(int C) {
     return cap > 1024 ? 1024 : cap;
 }
 
-// The sweep's tiles run on MFMA at every width, but for fp32 rows that are no
-// multiple of 8 and too wide for the re-rank (their lists come from the SIMT
-// tiles, which need none).
+// The sweep's tiles run on MFMA, but for fp32 rows that are no multiple of 8 and
+// either too wide for the re-rank (their lists come from the SIMT tiles, which need
+// none) or narrower than 64.  Such rows are split into three fp16 parts, 2^-22 of a
+// factor; near pairs' scores against float64 (rms, in 2^-24 of the rows' lengths;
+// the SIMT tiles' fp32 sums in brackets): d = 3 0.92 [0.42], 9 0.96 [0.66], 25 1.06
+// [1.10], 50 1.28 [1.54], 65 1.43 [1.71], 201 2.35 [3.05], 1,001 5.33 [6.97]; random
+// pairs' at 50 0.474 [0.463], 65 0.494 [0.494], 100 0.544 [0.573].  From 64 on the
+// matrix cores' shorter chains of sums give back more than the split takes.
 constexpr int kRerankMax = 16384;
+constexpr int kSplitMin = 64;
 bool use_mfma(int dim, int x_dtype) {
-    return x_dtype == SWANN_DTYPE_F16 || dim % 8 == 0 || dim <= kRerankMax;
+    return x_dtype == SWANN_DTYPE_F16 || dim % 8 == 0 || (dim >= kSplitMin && dim <= kRerankMax);
 }
 
 // An fp32 corpus on the MFMA path is swept on an fp16 screen and its lists

@@ -2321,8 +2321,8 @@ inline int64_t al256(int64_t b) { return ((b + 255) / 256) * 256; }
 // corpus of such a width is its own plane; another width is copied, zero past
 // the row's end.  An fp32 corpus is rounded to fp16 (a screen), except at widths
 // that are no multiple of 8, where the sweep has always ranked in fp32: those
-// take three parts a row (split3_rows), so their lists are chosen to fp32
-// accuracy still.
+// take three parts a row (split3_rows), each factor to 2^-22.  From the width where
+// they come here (use_mfma) their scores are no further from float64 than fp32 sums.
 inline bool plane_split3(int dim, int x_dtype) {
     return x_dtype == SWANN_DTYPE_F32 && dim % 8 != 0;
 }

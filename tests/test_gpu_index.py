@@ -1056,3 +1056,22 @@ def test_sweep_lists_do_not_depend_on_the_rows_scale(d, power):
     # products below the normal range lose bits, so a distance may move by an ulp
     assert torch.allclose(gd * 2.0 ** -power * 2.0 ** -power, wd, rtol=1e-6, atol=0)
     assert (gi != wi).float().mean() < 1e-3
+
+
+@pytest.mark.parametrize("d", [1, 3, 33, 63])
+def test_narrow_fp32_rows_are_ranked_by_fp32_sums(d):
+    """512 rows (v, 0, ..), v = 1 + k 2^-23 for consecutive k, and the longest lists,
+    which leave the exact re-rank no slack: each list is the 256 largest products
+    up to what an fp32 sum may turn, 2 u of the product a score (u = 2^-24: the
+    product's rounding and the distance's), so 4 u between two."""
+    n, C = 512, 256
+    v = 1 + torch.arange(12288 - n // 2, 12288 + n // 2, dtype=torch.float64) * 2.0 ** -23
+    v = v[torch.randperm(n, generator=torch.Generator().manual_seed(d))]
+    X = torch.zeros((n, d))
+    X[:, 0] = v.float()
+    gi, _ = B.knn_candidates(X.cuda(), C, metric="ip")
+    S = v[:, None] * v[None]
+    S.fill_diagonal_(-1)
+    kth = torch.topk(S, C, dim=1).values[:, -1]
+    got = S.gather(1, gi.cpu().long()).min(1).values
+    assert (kth - got).max() <= 4.01 * 2.0 ** -24 * float(S.max())
