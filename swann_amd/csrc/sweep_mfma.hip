@@ -2406,6 +2406,23 @@ inline bool sweep_sym(int64_t ntile) {
     return ntile >= 32;
 }
 
+// Whether the symmetric sweep looks for clusters and, where the rows form some,
+// runs in the locality order: by default from 192 row panels (n > 48,896), whenever
+// sweep_sym = 1 forces the symmetric sweep.  Order, bounds and their read-backs cost
+// about 2 ms however few the tiles left.  Gaussian mixtures of 8 to n / 700 clusters,
+// C = 128, ordered against the circle in the rows' order, in ms (fp16 768 wide; fp16
+// 128; fp32 1,536): 8,000 rows 1.87 to 2.14 against 0.86 (one-sided 1.12); 24,000
+// 2.7 to 2.9 against 2.2; 1.7 to 2.0 against 2.0; 5.8 to 6.5 against 4.4 to 5.0;
+// 40,000 3.2 to 3.9 against 4.1; 2.1 to 2.8 against 3.7; 7.6 to 9.6 against 8.0 to
+// 9.8; 49,200 3.4 to 4.4 against 5.6; 2.2 to 3.1 against 5.0; 8.2 to 11.6 against
+// 10.7 to 13.3; 200,000 8.6 to 18.9 against 56.  Rows stored cluster by cluster are
+// in a locality order already, which the check does not see: there the circle stays
+// ahead to 100,000 or so (60,000 x 768 fp16: 7.2 against 3.9, one-sided 14.3).
+constexpr int64_t kOrderPanels = 192;
+inline bool sweep_orders(int64_t ntile) {
+    return ntile > 2 * kSeedBand && (ntile >= kOrderPanels || option(kOptSweepSym) == 1);
+}
+
 // The symmetric sweep reads its overflow count back, which a stream under graph
 // capture cannot: there the one-sided sweep runs.
 inline bool capturing(hipStream_t st) {
@@ -2596,7 +2613,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
             int32_t* rid = nullptr;
             int32_t* rcnt = nullptr;
             const int32_t* ordered = nullptr;
-            if (ntile > 2 * kSeedBand && !split3 && !option_on(kOptSweepNoseed)) {
+            if (sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed)) {
                 bool clustered = false;
                 // the order's workspace (seed_bytes, repair_bytes)
                 float* sk = (float*)extra; extra += al256(n * kSketch * 4);
@@ -3051,7 +3068,7 @@ int64_t sweep_mfma_extra_bytes(int64_t n, int xdim, int x_dtype) {
     // run never finds less than it needs: a corpus the clustering check
     // declines at run time, or option sweep_noseed, still reserves it)
     const int64_t ntile = (n + kBM2 - 1) / kBM2;
-    const bool seeded = !plane_split3(xdim, x_dtype) && sweep_sym(ntile) && ntile > 2 * kSeedBand;
+    const bool seeded = !plane_split3(xdim, x_dtype) && sweep_sym(ntile) && sweep_orders(ntile);
     return base + (seeded ? seed_bytes(n, dim) + repair_bytes(1024) : 0);   // cap <= 1024
 }
 

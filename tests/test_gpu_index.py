@@ -1075,3 +1075,22 @@ def test_narrow_fp32_rows_are_ranked_by_fp32_sums(d):
     kth = torch.topk(S, C, dim=1).values[:, -1]
     got = S.gather(1, gi.cpu().long()).min(1).values
     assert (kth - got).max() <= 4.01 * 2.0 ** -24 * float(S.max())
+
+
+@pytest.mark.parametrize("n,ordered", [(9000, False), (48896, False), (48897, True)])
+def test_clustered_rows_are_ordered_only_where_it_pays(opt, n, ordered):
+    """A mixture of 8 clusters: below 192 row panels the sweep goes round the
+    circle, every tile once; from there it leaves out what the clusters' bounds
+    show empty.  Both give the one-sided sweep's lists."""
+    from swann_amd import _lib
+    g = torch.Generator().manual_seed(n)
+    X = 3 * torch.randn((8, 64), generator=g)[torch.randint(0, 8, (n,), generator=g)]
+    X = (X + torch.randn((n, 64), generator=g)).half().cuda()
+    nt = (n + 255) // 256
+    gi, gd = B.knn_candidates(X, 32, metric="l2")
+    tiles = int(_lib.lib().swann_sweep_tiles_scored())
+    assert tiles < nt * (nt + 1) // 3 if ordered else tiles == nt * (nt + 1) // 2
+    opt(sweep_sym=0)
+    wi, wd = B.knn_candidates(X, 32, metric="l2")
+    assert torch.equal(gd, wd)
+    assert (gi != wi).float().mean() < 1e-3            # ids swap only where distances tie
