@@ -255,14 +255,20 @@ int swann_select_nearest_noalloc(const float* Q, int64_t nq, int dim, const floa
  * scores come from fp16 MFMA tiles (fp16 corpus: exact products; fp32 corpus:
  * a power-of-two row-scaled fp16 screen keeps C+32 per row, which are then
  * re-ranked with exact fp32 dot products); otherwise from fp32 SIMT tiles.
- * `workspace`: swann_sweep_workspace_size bytes. */
+ * `workspace`: swann_sweep_workspace_size bytes.
+ * The call waits for the GPU (small read-backs) where it must choose: for an fp32
+ * corpus with dim % 8 == 0 (the rows' range), and from 192 row panels of 256 unless
+ * fp32 rows are no multiple of 8 (the clustering, the locality order, the repair).
+ * Elsewhere it only launches.  Under stream capture a sweep that may order its
+ * rows is recorded one-sided; an fp32 corpus with dim % 8 == 0 cannot be captured. */
 int64_t swann_sweep_workspace_size(int64_t n, int dim, int x_dtype, int C);
 int swann_build_sweep(const void* X, int x_dtype, int64_t n, int dim, int metric, int C,
                       int32_t* cand, float* cdist, void* workspace, void* stream);
 
 /* Tiles of 256 x 256 rows the last swann_build_sweep on this thread scored
  * on MFMA (the symmetric sweep's bands, less the tiles the locality-ordered
- * sweep proved empty, plus any repair); -1 before any sweep.  No counterpart
+ * sweep proved empty, plus any repair the host launched; not those of panels
+ * the device chose to sweep again); -1 before any sweep.  No counterpart
  * in the reference (its sweep scores every pair): a diagnostic for the
  * executed-FLOP figure of the bench (2 * 256 * 256 * dim FLOP a tile). */
 int64_t swann_sweep_tiles_scored(void);

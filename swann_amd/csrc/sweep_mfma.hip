@@ -256,6 +256,9 @@ struct MfmaSweepArgs {
     // second list overflowed): workgroup g takes panel plist[g / G]
     const int* plist;
     int npl;
+    // one-sided sweep of the row panels that hold a flagged row: the workgroups of
+    // the others end at once
+    const int* pflag;
     // the pruned ordered sweep: workgroup (panel) I scores only the column
     // tiles tlist[I * kBandMax + k], k < tcnt[I] (ascending, inside its band);
     // a one-sided launch over listed panels (the bounded repair): panel
@@ -909,6 +912,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
                           : (int)xcd_remap(blockIdx.x, (int64_t)(a.plist ? a.npl : ntile) * G);
     const int r0 = (a.sym ? lid : a.plist ? a.plist[lid / G] : lid / G) * kBM2;
     const int split = a.sym ? 0 : lid % G;
+    if (a.pflag &&
+        !__syncthreads_or(tid < kBM2 && r0 + tid < n ? a.pflag[r0 + tid] : 0)) return;
 
     // a score is (row scale * sum) * column scale; the three parts' sums reach
     // 2^30 a product, which the row's scale takes back first, so that nothing
@@ -2335,7 +2340,7 @@ inline int64_t prune_bytes(int64_t n, int dim);
 
 inline int64_t seed_bytes(int64_t n, int dim) {
     const int64_t ntile = (n + kBM2 - 1) / kBM2;
-    return al256(n * kSketch * 4) + al256(n * 4) * 7 + al256(kMaxPivots * 4) +
+    return al256(n * kSketch * 4) + al256(n * 4) * 6 + al256(kMaxPivots * 4) +
            al256(n * (int64_t)dim * 2) + al256(ntile * 4) + 256 +
            al256((int64_t)kMaxPivots * kSketch * 4) + al256((kMaxPivots + 1) * 4) +
            al256((int64_t)kMaxPivots * kMaxPivots * 4) + al256(kMaxPivots * 4) +
@@ -2423,8 +2428,8 @@ inline bool sweep_orders(int64_t ntile) {
     return ntile > 2 * kSeedBand && (ntile >= kOrderPanels || option(kOptSweepSym) == 1);
 }
 
-// The symmetric sweep reads its overflow count back, which a stream under graph
-// capture cannot: there the one-sided sweep runs.
+// A sweep that may order the rows reads the clustering and an overflow count back,
+// which a stream under graph capture cannot: there the one-sided sweep runs.
 inline bool capturing(hipStream_t st) {
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &c) != hipSuccess) {
@@ -2516,7 +2521,8 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
     const bool off32 = (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32);
     if ((uintptr_t)hi % 16 == 0 && off32 && (split3 || !option_on(kOptSweepRegstage))) {
         const int64_t ntile = (n + kBM2 - 1) / kBM2;
-        if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !capturing(st)) {
+        const bool orders = sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed);
+        if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !(orders && capturing(st))) {
             // symmetric sweep: tile (I, J), J >= I, scored once for the rows of
             // both panels; launched in bands of J - I (1, 1, 2, 4, ... 256, then
             // kBandMax at a time) with a merge after each, so every launch
@@ -2525,6 +2531,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
             float* gthr = (float*)extra; extra += al256(n * 4);
             int* ovf = (int*)extra; extra += 256;
             int* mcnt = (int*)extra; extra += al256(n * 4);
+            int* flag = (int*)extra; extra += al256(n * 4);      // rows whose second list overflowed
             MfmaSweepArgs s = a;
             s.splits = 2;
             s.sym = 1;
@@ -2606,14 +2613,14 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
             };
             const unsigned nb256 = (unsigned)((n + 255) / 256);
             float* seed = nullptr;
-            int* flag = nullptr;         // rows whose second list overflowed (ordered sweep)
+            hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
             int* plist = nullptr;
             int* npl = nullptr;
             float* rkey = nullptr;       // the few-panel repair's scratch lists
             int32_t* rid = nullptr;
             int32_t* rcnt = nullptr;
             const int32_t* ordered = nullptr;
-            if (sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed)) {
+            if (orders) {
                 bool clustered = false;
                 // the order's workspace (seed_bytes, repair_bytes)
                 float* sk = (float*)extra; extra += al256(n * kSketch * 4);
@@ -2624,7 +2631,6 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 float* scp = (float*)extra; extra += al256(n * 4) * 2;
                 int* pcnt = (int*)extra; extra += al256(kMaxPivots * 4);
                 _Float16* hp = (_Float16*)extra; extra += al256(n * (int64_t)dim * 2);
-                flag = (int*)extra; extra += al256(n * 4);
                 plist = (int*)extra; extra += al256(ntile * 4);
                 npl = (int*)extra; extra += 256;
                 float* psk = (float*)extra; extra += al256((int64_t)kMaxPivots * kSketch * 4);
@@ -2723,18 +2729,13 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                                        perm);
                 }
                 if (!clustered) {
-                    // not clustered: the rows' own order, no seeds; the flags
-                    // name the rows to repair
-                    seed = nullptr;
-                    hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
+                    seed = nullptr;              // the rows' own order, no seeds
                     goto plain;
                 }
                 hipLaunchKernelGGL(gather_rows, dim3(nrb), dim3(256), 0, st, hi, n, dim, perm, xn,
                                    scaled ? scale : nullptr, hp, xnp, scp);
                 hipLaunchKernelGGL(sym_init, dim3(nb256), dim3(256), 0, st, gthr, bcnt, ovf, n,
                                    (const float*)nullptr, mcnt);
-                if (in_order)
-                    hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
                 MfmaSweepArgs pre = s;
                 pre.hi = hp;
                 pre.cols = hp;
@@ -2861,7 +2862,6 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 } else {
                     hipLaunchKernelGGL(seed_map, dim3(nb256), dim3(256), 0, st, gthr, perm, xn, n,
                                        seed);
-                    flag = nullptr;
                 }
             }
         plain:
@@ -2871,10 +2871,29 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 const int rc = bands(s, 0, ntile / 2 + 1, seed, flag, false, true);
                 if (rc) return rc;
             }
+            if (!orders) {
+                // a list that overflowed lost candidates: its panel is swept again
+                // the one-sided way, chosen on the device (nothing is read back, so
+                // the call returns while the GPU works, and can be captured)
+                MfmaSweepArgs rep = s;
+                rep.sym = 0;
+                rep.wrap = 0;
+                rep.pflag = flag;
+                const unsigned rg = (unsigned)(ntile * 2);
+                if (scaled) {
+                    if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                    else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                } else {
+                    if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                    else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                }
+                g_tiles_scored += host_tiles;
+                *used = 2;
+                return launch_status("sweep (mfma, circle repair)");
+            }
         swept:
-            // a list that overflowed lost candidates: sweep its panel again
-            // the one-sided way, or without flags every panel (one small
-            // read-back; the build is not on the search path)
+            // the same where the host has read the clustering back already, so
+            // the panels' count can choose how they are swept
             int dropped = 0;
             unsigned long long pruned_kept = 0;
             if (hipMemcpyAsync(&dropped, ovf, sizeof(int), hipMemcpyDeviceToHost, st) !=
@@ -2891,135 +2910,133 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 *perm_out = ordered;
                 return SWANN_OK;
             }
-            if (ordered || flag) {
-                // the repair: the row panels holding a row
-                // whose second list overflowed are swept again one-sided
-                // (two column halves, lists 0 and 1 of each row written from
-                // scratch), so those rows' lists are exact again
-                hipLaunchKernelGGL(fill_zero, dim3(1), dim3(256), 0, st, npl, 1);
-                hipLaunchKernelGGL(flag_panels, dim3((unsigned)((ntile + 255) / 256)), dim3(256), 0,
-                                   st, flag, n, (int)ntile, plist, npl);
-                int np = 0;
-                if (hipMemcpyAsync(&np, npl, sizeof(int), hipMemcpyDeviceToHost, st) !=
+            // the repair: the row panels holding a row
+            // whose second list overflowed are swept again one-sided
+            // (two column halves, lists 0 and 1 of each row written from
+            // scratch), so those rows' lists are exact again
+            hipLaunchKernelGGL(fill_zero, dim3(1), dim3(256), 0, st, npl, 1);
+            hipLaunchKernelGGL(flag_panels, dim3((unsigned)((ntile + 255) / 256)), dim3(256), 0,
+                               st, flag, n, (int)ntile, plist, npl);
+            int np = 0;
+            if (hipMemcpyAsync(&np, npl, sizeof(int), hipMemcpyDeviceToHost, st) !=
+                    hipSuccess ||
+                hipStreamSynchronize(st) != hipSuccess) {
+                set_error("sweep (mfma, symmetric): reading the repair count failed");
+                return SWANN_E_LAUNCH;
+            }
+            SWANN_REQUIRE(np >= 1 && np <= ntile, "sweep: repair panel count out of range");
+            // With the pruned sweep's groups, a repaired panel sweeps only
+            // the tiles some row of it can still need, each row against
+            // every group at its own threshold (repair_need).  The marks,
+            // the rows' stats and the lists take the bands' list space.
+            const int* rlist = nullptr;
+            const int* rlcnt = nullptr;
+            int64_t rtiles = (int64_t)np * ntile;
+            const int64_t rspace = 2 * (int64_t)np * ntile + 4 * (int64_t)np * kBM2;
+            if (tlb && rcen && rng > 0 && rspace <= ntile * kBandMax) {
+                int* rneed = tlist + (int64_t)np * ntile;
+                double* rst = (double*)(tlist + 2 * (int64_t)np * ntile);
+                hipLaunchKernelGGL(fill_u32, dim3((unsigned)((np * ntile + 255) / 256)),
+                                   dim3(256), 0, st, (unsigned*)rneed, (int64_t)np * ntile, 0u);
+                hipLaunchKernelGGL(repair_row_stats, dim3((unsigned)np), dim3(256), 0, st, rhp,
+                                   rscp, rxnp, (const int*)plist, n, dim, scaled, rst);
+                hipLaunchKernelGGL(repair_need,
+                                   dim3((unsigned)((rng + kGB - 1) / kGB), kBM2 / kGB,
+                                        (unsigned)np),
+                                   dim3(256), 0, st, rhp, rscp, rcen, rpst, rglist, rng,
+                                   (const float*)gthr, (const int*)plist,
+                                   (const double*)rst, n, (int)ntile, dim, metric, scaled,
+                                   rneed);
+                hipLaunchKernelGGL(fill_zero, dim3(1), dim3(256), 0, st, (int*)tsum, 2);
+                hipLaunchKernelGGL(repair_list, dim3((unsigned)np), dim3(64), 0, st,
+                                   (const int*)rneed, (const int*)plist, (int)ntile, tlist,
+                                   tcnt, tsum);
+                unsigned long long rt = 0;
+                if (hipMemcpyAsync(&rt, tsum, sizeof(rt), hipMemcpyDeviceToHost, st) !=
                         hipSuccess ||
                     hipStreamSynchronize(st) != hipSuccess) {
-                    set_error("sweep (mfma, symmetric): reading the repair count failed");
+                    set_error("sweep (mfma, symmetric): reading the repair tile count failed");
                     return SWANN_E_LAUNCH;
                 }
-                SWANN_REQUIRE(np >= 1 && np <= ntile, "sweep: repair panel count out of range");
-                // With the pruned sweep's groups, a repaired panel sweeps only
-                // the tiles some row of it can still need, each row against
-                // every group at its own threshold (repair_need).  The marks,
-                // the rows' stats and the lists take the bands' list space.
-                const int* rlist = nullptr;
-                const int* rlcnt = nullptr;
-                int64_t rtiles = (int64_t)np * ntile;
-                const int64_t rspace = 2 * (int64_t)np * ntile + 4 * (int64_t)np * kBM2;
-                if (tlb && rcen && rng > 0 && rspace <= ntile * kBandMax) {
-                    int* rneed = tlist + (int64_t)np * ntile;
-                    double* rst = (double*)(tlist + 2 * (int64_t)np * ntile);
-                    hipLaunchKernelGGL(fill_u32, dim3((unsigned)((np * ntile + 255) / 256)),
-                                       dim3(256), 0, st, (unsigned*)rneed, (int64_t)np * ntile, 0u);
-                    hipLaunchKernelGGL(repair_row_stats, dim3((unsigned)np), dim3(256), 0, st, rhp,
-                                       rscp, rxnp, (const int*)plist, n, dim, scaled, rst);
-                    hipLaunchKernelGGL(repair_need,
-                                       dim3((unsigned)((rng + kGB - 1) / kGB), kBM2 / kGB,
-                                            (unsigned)np),
-                                       dim3(256), 0, st, rhp, rscp, rcen, rpst, rglist, rng,
-                                       (const float*)gthr, (const int*)plist,
-                                       (const double*)rst, n, (int)ntile, dim, metric, scaled,
-                                       rneed);
-                    hipLaunchKernelGGL(fill_zero, dim3(1), dim3(256), 0, st, (int*)tsum, 2);
-                    hipLaunchKernelGGL(repair_list, dim3((unsigned)np), dim3(64), 0, st,
-                                       (const int*)rneed, (const int*)plist, (int)ntile, tlist,
-                                       tcnt, tsum);
-                    unsigned long long rt = 0;
-                    if (hipMemcpyAsync(&rt, tsum, sizeof(rt), hipMemcpyDeviceToHost, st) !=
-                            hipSuccess ||
-                        hipStreamSynchronize(st) != hipSuccess) {
-                        set_error("sweep (mfma, symmetric): reading the repair tile count failed");
-                        return SWANN_E_LAUNCH;
-                    }
-                    SWANN_REQUIRE(rt >= (unsigned long long)np &&
-                                      rt <= (unsigned long long)np * (unsigned long long)ntile,
-                                  "sweep: repair tile count out of range");
-                    rtiles = (int64_t)rt;
-                    rlist = tlist;
-                    rlcnt = tcnt;
-                }
-                // panels repaired one at a time, 16 ways (option sweep_repair_max)
-                const int rmax = option(kOptSweepRepairMax);
-                if (np <= rmax && C * kRepairSplits <= kRepairSort) {
-                    std::vector<int> ph(np);
-                    if (hipMemcpyAsync(ph.data(), plist, (size_t)np * 4, hipMemcpyDeviceToHost,
-                                       st) != hipSuccess ||
-                        hipStreamSynchronize(st) != hipSuccess) {
-                        set_error("sweep (mfma, symmetric): reading the repair panels failed");
-                        return SWANN_E_LAUNCH;
-                    }
-                    g_tiles_scored += rtiles;
-                    for (int i = 0; i < np; ++i) {
-                        SWANN_REQUIRE(ph[i] >= 0 && ph[i] < ntile, "sweep: repair panel out of range");
-                        // the one-sided sweep of panel ph[i] into the scratch:
-                        // its list addresses are row-absolute, so the bases
-                        // are shifted by the panel's first row (only rows of
-                        // this panel are touched)
-                        const int64_t rb = (int64_t)ph[i] * kBM2;
-                        MfmaSweepArgs rep = s;
-                        rep.sym = 0;
-                        rep.wrap = 0;
-                        rep.splits = kRepairSplits;
-                        rep.plist = plist + i;
-                        rep.npl = 1;
-                        rep.tlist = rlist ? rlist + (int64_t)i * ntile : nullptr;
-                        rep.tcnt = rlist ? rlcnt + i : nullptr;
-                        rep.tstride = (int)ntile;
-                        rep.bkey = rkey - rb * kRepairSplits * cap;
-                        rep.bid = rid - rb * kRepairSplits * cap;
-                        rep.bcnt = rcnt - rb * kRepairSplits;
-                        const unsigned rg = (unsigned)kRepairSplits;
-                        if (scaled) {
-                            if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                            else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                        } else {
-                            if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                            else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                        }
-                        hipLaunchKernelGGL(repair_merge, dim3(kBM2), dim3(256), 0, st,
-                                           (const float*)rkey, (const int32_t*)rid,
-                                           (const int32_t*)rcnt, (int)rb, n, cap, C, ordered, bkey,
-                                           bid, bcnt);
-                        const int rc = launch_status("sweep (mfma, ordered repair)");
-                        if (rc) return rc;
-                    }
-                    *used = 2;
-                    *perm_out = ordered;
-                    return SWANN_OK;
+                SWANN_REQUIRE(rt >= (unsigned long long)np &&
+                                  rt <= (unsigned long long)np * (unsigned long long)ntile,
+                              "sweep: repair tile count out of range");
+                rtiles = (int64_t)rt;
+                rlist = tlist;
+                rlcnt = tcnt;
+            }
+            // panels repaired one at a time, 16 ways (option sweep_repair_max)
+            const int rmax = option(kOptSweepRepairMax);
+            if (np <= rmax && C * kRepairSplits <= kRepairSort) {
+                std::vector<int> ph(np);
+                if (hipMemcpyAsync(ph.data(), plist, (size_t)np * 4, hipMemcpyDeviceToHost,
+                                   st) != hipSuccess ||
+                    hipStreamSynchronize(st) != hipSuccess) {
+                    set_error("sweep (mfma, symmetric): reading the repair panels failed");
+                    return SWANN_E_LAUNCH;
                 }
                 g_tiles_scored += rtiles;
-                MfmaSweepArgs rep = s;
-                rep.sym = 0;
-                rep.wrap = 0;
-                rep.splits = 2;
-                rep.plist = plist;
-                rep.npl = np;
-                rep.tlist = rlist;
-                rep.tcnt = rlcnt;
-                rep.tstride = (int)ntile;
-                const unsigned rg = (unsigned)(np * 2);
-                if (scaled) {
-                    if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                    else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                } else {
-                    if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
-                    else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                for (int i = 0; i < np; ++i) {
+                    SWANN_REQUIRE(ph[i] >= 0 && ph[i] < ntile, "sweep: repair panel out of range");
+                    // the one-sided sweep of panel ph[i] into the scratch:
+                    // its list addresses are row-absolute, so the bases
+                    // are shifted by the panel's first row (only rows of
+                    // this panel are touched)
+                    const int64_t rb = (int64_t)ph[i] * kBM2;
+                    MfmaSweepArgs rep = s;
+                    rep.sym = 0;
+                    rep.wrap = 0;
+                    rep.splits = kRepairSplits;
+                    rep.plist = plist + i;
+                    rep.npl = 1;
+                    rep.tlist = rlist ? rlist + (int64_t)i * ntile : nullptr;
+                    rep.tcnt = rlist ? rlcnt + i : nullptr;
+                    rep.tstride = (int)ntile;
+                    rep.bkey = rkey - rb * kRepairSplits * cap;
+                    rep.bid = rid - rb * kRepairSplits * cap;
+                    rep.bcnt = rcnt - rb * kRepairSplits;
+                    const unsigned rg = (unsigned)kRepairSplits;
+                    if (scaled) {
+                        if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                        else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                    } else {
+                        if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                        else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                    }
+                    hipLaunchKernelGGL(repair_merge, dim3(kBM2), dim3(256), 0, st,
+                                       (const float*)rkey, (const int32_t*)rid,
+                                       (const int32_t*)rcnt, (int)rb, n, cap, C, ordered, bkey,
+                                       bid, bcnt);
+                    const int rc = launch_status("sweep (mfma, ordered repair)");
+                    if (rc) return rc;
                 }
-                const int rc = launch_status("sweep (mfma, ordered repair)");
-                if (rc) return rc;
                 *used = 2;
                 *perm_out = ordered;
                 return SWANN_OK;
             }
+            g_tiles_scored += rtiles;
+            MfmaSweepArgs rep = s;
+            rep.sym = 0;
+            rep.wrap = 0;
+            rep.splits = 2;
+            rep.plist = plist;
+            rep.npl = np;
+            rep.tlist = rlist;
+            rep.tcnt = rlcnt;
+            rep.tstride = (int)ntile;
+            const unsigned rg = (unsigned)(np * 2);
+            if (scaled) {
+                if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 1, 16>), dim3(rg), dim3(1024), 0, st, rep);
+            } else {
+                if (ip) hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_IP, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+                else hipLaunchKernelGGL((sweep_dma_kernel<SWANN_METRIC_L2, 0, 16>), dim3(rg), dim3(1024), 0, st, rep);
+            }
+            const int rc = launch_status("sweep (mfma, ordered repair)");
+            if (rc) return rc;
+            *used = 2;
+            *perm_out = ordered;
+            return SWANN_OK;
         }
         a.splits = splits;
         *used = splits;
@@ -3061,7 +3078,7 @@ int64_t sweep_mfma_extra_bytes(int64_t n, int xdim, int x_dtype) {
     const int64_t planes = plane_split3(xdim, x_dtype) ? 2
                            : x_dtype == SWANN_DTYPE_F16 && dim == xdim ? 0 : 1;
     const int64_t base = al256(n * 4) * 2 + planes * al256(n * (int64_t)dim * 2) +
-                         al256(n * 4) + 256 + al256(n * 4);
+                         al256(n * 4) + 256 + al256(n * 4) * 2;
     // the locality order, seeds and panel repair run only in the symmetric
     // direct-load sweep past its seed bands; only a sweep that may take that
     // path reserves their scratch (a superset of the run's conditions, so the

@@ -945,9 +945,8 @@ def test_symmetric_sweep_around_the_circle(opt, n, dtype, metric, d):
 
 
 def test_fp16_sweep_under_graph_capture():
-    """A stream under capture cannot read the symmetric sweep's overflow count
-    back: the sweep is recorded one-sided, and every replay equals the eager
-    one."""
+    """The symmetric sweep and its repair record nothing that a stream under capture
+    cannot: every replay equals the eager sweep."""
     X = torch.from_numpy(gaussian(9000, 128, 5, True)).cuda().half()
     wi, wd = B.knn_candidates(X, 32)
     side = torch.cuda.Stream()
@@ -1094,3 +1093,75 @@ def test_clustered_rows_are_ordered_only_where_it_pays(opt, n, ordered):
     wi, wd = B.knn_candidates(X, 32, metric="l2")
     assert torch.equal(gd, wd)
     assert (gi != wi).float().mean() < 1e-3            # ids swap only where distances tie
+
+
+@pytest.mark.parametrize("d,dtype", [(128, "f16"), (100, "f16"), (100, "f32")])
+def test_symmetric_sweep_returns_before_the_gpu_is_done(d, dtype):
+    """Rows too few to be ordered: the call reads nothing back, so it returns while
+    work queued ahead of it still runs, and its lists are the same."""
+    X = torch.from_numpy(gaussian(9000, d, d, True)).cuda()
+    X = X.half() if dtype == "f16" else X
+    wi, wd = B.knn_candidates(X, 64)
+    A = torch.randn((8192, 8192), device="cuda")
+    Y = torch.empty_like(A)
+    torch.mm(A, A, out=Y)
+    torch.cuda.synchronize()
+    ahead = torch.cuda.Event()
+    for _ in range(40):                                # a few hundred milliseconds
+        torch.mm(A, A, out=Y)
+    ahead.record()
+    gi, gd = B.knn_candidates(X, 64)
+    early = not ahead.query()
+    torch.cuda.synchronize()
+    assert early
+    assert torch.equal(gd, wd)
+    assert (gi != wi).float().mean() < 1e-3
+
+
+@pytest.mark.parametrize("n", [9000, 49200])
+@pytest.mark.parametrize("d,dtype", [(64, "f16"), (100, "f32")])
+def test_sweep_of_any_size_under_graph_capture(n, d, dtype):
+    """Sizes whose rows may be ordered (recorded one-sided) and widths swept as three
+    parts a row."""
+    X = torch.from_numpy(gaussian(n, d, 5, True)).cuda()
+    X = X.half() if dtype == "f16" else X
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        wi, wd = B.knn_candidates(X, 32)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gi, gd = B.knn_candidates(X, 32)
+    for _ in range(3):
+        gi.zero_()
+        gd.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gd, wd)
+        assert (gi != wi).float().mean() < 1e-3
+        B.knn_candidates(X, 32)
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("d", [64, 100, 320])
+@pytest.mark.parametrize("fcap", [1, 60, 110])
+def test_only_overflowed_panels_are_swept_again(opt, d, fcap):
+    """Second lists with little room: some rows' overflow or all do, at widths of one
+    part and of three.  The panels that hold one are swept again, nothing else is
+    (the tiles the launches scored are the circle's), and the lists are the
+    one-sided sweep's."""
+    from swann_amd import _lib
+    n, C = 8500, 64
+    nt = (n + 255) // 256
+    X = torch.from_numpy(gaussian(n, d, d, True)).cuda()
+    # rows 0..999 near one another and stored far apart: their lists' owners differ
+    X[torch.arange(0, 8000, 8)] = X[0] + 0.01 * X[torch.arange(0, 8000, 8)]
+    opt(sweep_sym=0)
+    wi, wd = B.knn_candidates(X, C)
+    opt(sweep_sym=1, sweep_noseed=1, sweep_sym_fcap=fcap)
+    gi, gd = B.knn_candidates(X, C)
+    assert int(_lib.lib().swann_sweep_tiles_scored()) == nt * (nt + 1) // 2
+    assert torch.allclose(gd, wd, rtol=1e-6, atol=1e-6)
+    assert (gi != wi).float().mean() < 2e-3
