@@ -1068,23 +1068,31 @@ int sweep_cap(int C) {
 // [1.10], 50 1.28 [1.54], 65 1.43 [1.71], 201 2.35 [3.05], 1,001 5.33 [6.97]; random
 // pairs' at 50 0.474 [0.463], 65 0.494 [0.494], 100 0.544 [0.573].  From 64 on the
 // matrix cores' shorter chains of sums give back more than the split takes.
+// And but for corpora so small that the SIMT tiles never cut a list (n <= C + 448),
+// at ragged widths with few products, C = 128, in ms, SIMT against MFMA: fp16 150 x
+// 33 0.047 to 0.055, 300 x 33 0.078 to 0.100, 480 x 33 0.107 to 0.100, 300 x 65 0.102
+// to 0.101; fp32 (whose MFMA lists are re-ranked) 150 x 201 0.115 to 0.131, 300 x 150
+// 0.157 to 0.17, 480 x 100 0.178 to 0.18, 576 x 100 0.223 to 0.205.
 constexpr int kRerankMax = 16384;
 constexpr int kSplitMin = 64;
-bool use_mfma(int dim, int x_dtype) {
-    return x_dtype == SWANN_DTYPE_F16 || dim % 8 == 0 || (dim >= kSplitMin && dim <= kRerankMax);
+bool use_mfma(int64_t n, int dim, int x_dtype, int C) {
+    const bool f32 = x_dtype == SWANN_DTYPE_F32;
+    if (dim % 8 == 0) return true;
+    if (n <= sweep_cap(C) - kCT && n * dim <= (f32 ? 48000 : 12000)) return false;
+    return !f32 || (dim >= kSplitMin && dim <= kRerankMax);
 }
 
 // An fp32 corpus on the MFMA path is swept on an fp16 screen and its lists
 // re-ranked in exact fp32; fp16 corpora and the fp32 SIMT sweep are exact.
-bool screened(int x_dtype, int dim) {
-    return x_dtype == SWANN_DTYPE_F32 && use_mfma(dim, x_dtype);
+bool screened(int64_t n, int dim, int x_dtype, int C) {
+    return x_dtype == SWANN_DTYPE_F32 && use_mfma(n, dim, x_dtype, C);
 }
 
 // Candidates the fp32 screen keeps per row before the exact re-rank (at
 // least C: when C + 32 exceeds n or the sweep's list limit the screen keeps
 // what it can, and the re-rank still replaces every distance by the exact one).
 int screen_count(int C, int64_t n, int x_dtype, int dim) {
-    if (!screened(x_dtype, dim)) return C;
+    if (!screened(n, dim, x_dtype, C)) return C;
     int64_t cs = C + 32;
     if (cs > kMaxC) cs = kMaxC;
     if (cs > n) cs = n;
@@ -1103,11 +1111,12 @@ extern "C" {
 
 int64_t swann_sweep_workspace_size(int64_t n, int dim, int x_dtype, int C) {
     const int Cs = screen_count(C, n, x_dtype, dim);
-    const int cap = use_mfma(dim, x_dtype) ? sweep_mfma_cap(Cs) : sweep_cap(C);
-    const int64_t G = use_mfma(dim, x_dtype) ? sweep_mfma_splits(n) : 1;
+    const bool mf = use_mfma(n, dim, x_dtype, C);
+    const int cap = mf ? sweep_mfma_cap(Cs) : sweep_cap(C);
+    const int64_t G = mf ? sweep_mfma_splits(n) : 1;
     int64_t b = align256(n * 4) + align256(n * G * cap * 4) * 2 + align256(n * G * 4);
-    if (screened(x_dtype, dim)) b += align256(n * (int64_t)Cs * 4) * 2;
-    if (use_mfma(dim, x_dtype)) b += sweep_mfma_extra_bytes(n, dim, x_dtype);
+    if (screened(n, dim, x_dtype, C)) b += align256(n * (int64_t)Cs * 4) * 2;
+    if (mf) b += sweep_mfma_extra_bytes(n, dim, x_dtype);
     return b;
 }
 
@@ -1124,9 +1133,9 @@ int swann_build_sweep(const void* X, int x_dtype, int64_t n, int dim, int metric
     SWANN_REQUIRE(n <= INT32_MAX / 2, "sweep: n too large");
     SWANN_REQUIRE(X && cand && cdist && workspace, "sweep: a required pointer is NULL");
     hipStream_t st = (hipStream_t)stream;
-    const bool mf = use_mfma(dim, x_dtype);
+    const bool mf = use_mfma(n, dim, x_dtype, C);
     const int Cs = screen_count(C, n, x_dtype, dim);
-    const bool rerank = screened(x_dtype, dim);
+    const bool rerank = screened(n, dim, x_dtype, C);
     SWANN_REQUIRE(!rerank || dim <= kRerankMax, "sweep: dimension too large for the re-rank");
     const int cap = mf ? sweep_mfma_cap(Cs) : sweep_cap(C);
     const int G = mf ? sweep_mfma_splits(n) : 1;
@@ -1162,8 +1171,9 @@ int swann_build_sweep(const void* X, int x_dtype, int64_t n, int dim, int metric
         rc = launch_status("sweep");
     }
     if (rc) return rc;
-    // one list holds up to cap; G > 1 lists were each cut to Cs by the sweep
-    const int most = Gu > 1 ? Gu * Cs : cap;
+    // one list holds up to cap; G > 1 lists were each cut to Cs by the sweep, but
+    // where a whole row fits one (they then hold n - 1 together)
+    const int most = Gu > 1 ? (n <= cap ? (int)n : Gu * Cs) : cap;
     int np = 2;
     while (np < most) np <<= 1;
     if (!rerank) {

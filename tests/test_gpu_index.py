@@ -1165,3 +1165,33 @@ def test_only_overflowed_panels_are_swept_again(opt, d, fcap):
     assert int(_lib.lib().swann_sweep_tiles_scored()) == nt * (nt + 1) // 2
     assert torch.allclose(gd, wd, rtol=1e-6, atol=1e-6)
     assert (gi != wi).float().mean() < 2e-3
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("n,d,C", [(2, 5, 1), (2, 64, 2), (65, 7, 65), (240, 50, 20), (241, 50, 20),
+                                   (468, 25, 20), (469, 25, 20), (480, 100, 128), (481, 100, 128),
+                                   (576, 20, 128), (577, 20, 128), (704, 64, 224), (896, 72, 128),
+                                   (897, 72, 128), (832, 64, 32), (833, 64, 32), (788, 33, 20),
+                                   (789, 33, 20), (992, 16, 224), (1025, 16, 224),
+                                   (300, 16385, 8)])
+def test_sweep_of_small_corpora(n, d, C, dtype):
+    """Sizes on both sides of where a corpus's rows fit one list uncut (n = C + 448 on
+    the SIMT tiles, the room of a list on the matrix cores), where a ragged width
+    changes tiles, and a width past the re-rank's: the float64 top-C up to the
+    rounding of d products and sums."""
+    X = torch.from_numpy(gaussian(n, d, n + d, False))
+    X = X.half() if dtype == "f16" else X
+    for metric in ("ip", "l2"):
+        gi, gd = (t.cpu() for t in B.knn_candidates(X.cuda(), C, metric=metric))
+        x = X.double()
+        sq = (x * x).sum(1)
+        D = 1 - x @ x.T if metric == "ip" else (sq[:, None] + sq[None] - 2 * x @ x.T).clamp(min=0)
+        D.fill_diagonal_(3.4e38)                       # self comes after every other row
+        want = torch.topk(D, C, dim=1, largest=False).values
+        bound = (2 * d + 8) * 2.0 ** -24 * (1 + float(sq.max())) * 2
+        assert ((gi >= 0) & (gi < n)).all()
+        assert (gi.sort(1).values.diff(dim=1) > 0).all()
+        self_ = want > 1e38
+        assert torch.equal(gd > 1e38, self_)
+        assert ((gd.double() - want)[~self_].abs() <= bound).all()
+        assert ((D.gather(1, gi.long()) - want)[~self_].abs() <= 2 * bound).all()
