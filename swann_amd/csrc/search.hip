@@ -802,10 +802,10 @@ __device__ __forceinline__ void advance_body(const AdvArgs& a) {
         const int deg = (p >= 0 && p < a.n) ? D : 0;
         if (AHEAD && a.bound && wave == 0) ebound = load_agent_f(a.bound + q);
         if constexpr (EAGER) {
-            // claim bits and no visited table (checked by the dispatch)
-            for (int nidx = team; nidx < deg; nidx += NT) {
-                const int v = a.G[(int64_t)p * D + nidx];    // the same for the team
-                if (v < 0 || v >= a.n) continue;
+            // a team a neighbour, claim bits and no visited table (checked by the
+            // dispatch)
+            const int v = team < deg ? a.G[(int64_t)p * D + team] : -1;
+            if (v >= 0 && v < a.n) {                         // the same for the team
                 const uint32_t bit = 1u << (v & 31);
                 uint32_t old = 0u;
                 if (tl == 0)
@@ -819,7 +819,7 @@ __device__ __forceinline__ void advance_body(const AdvArgs& a) {
                         ++r_hits; ++cov;                        // owned elsewhere
                     } else {
                         ++r_claim; ++r_evals;
-                        c_id[nidx] = v; c_d[nidx] = d; c_l[nidx] = plin;
+                        c_id[team] = v; c_d[team] = d; c_l[team] = plin;
                     }
                 }
             }
@@ -1300,7 +1300,7 @@ bool rows_vec_ok(const void* X, int dim, int x_dtype) {
 // Workgroups of one advance_kernel instance a CU holds at once (registers
 // and LDS), from the runtime's occupancy query; 0 if the query fails.
 template <int TEAM, typename XT>
-int advance_occupancy(int block, size_t lds, bool codes) {
+int advance_occupancy(int block, size_t lds, bool codes, bool eager) {
     int v = 0;
     hipError_t e;
     if (block == 64)
@@ -1313,6 +1313,9 @@ int advance_occupancy(int block, size_t lds, bool codes) {
                         &v, advance_codes_kernel<TEAM, XT, 256>, 256, lds)
                   : hipOccupancyMaxActiveBlocksPerMultiprocessor(
                         &v, advance_kernel<TEAM, XT, 256>, 256, lds);
+    else if (eager)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, advance_eager_kernel<TEAM, XT>, 1024,
+                                                         lds);
     else
         e = codes ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
                         &v, advance_codes_kernel<TEAM, XT, 1024>, 1024, lds)
@@ -1322,14 +1325,23 @@ int advance_occupancy(int block, size_t lds, bool codes) {
 }
 
 // Whether the advance runs EAGER (advance_body): claim bits without a visited
-// table, sixteen waves a branch, and a graph row whose neighbours' vectors, read
-// whole by one CU each step, cost less than the round trip they save.  A search
-// of one query over 50,000 rows at degree 64, 32 branches: 24 KB a step (96
-// fp32) 210 to 184 us, 64 KB 217 to 206, 96 KB 223 to 218; 192 KB 242 to 256.
-bool advance_eager(const AdvArgs& a, int x_dtype, int block) {
+// table, sixteen waves a branch, a team for every neighbour (a second round of
+// neighbours is read, claimed or not, only after the first), and a graph row whose
+// neighbours' vectors, read whole by one CU each step, cost less than the round trip
+// they save.  Searches over 50,000 rows, 32 branches, listed to eager, in us:
+//   one query, degree 64, team 16: 24 KB a step (96 fp32) 210 to 184, 64 KB 217 to
+//   206, 96 KB 223 to 218; 192 KB 242 to 256
+//   96 fp32, teams 8 | 16 | 32 | 64: one query, degree 64 210 to 186 | 211 to 189 |
+//   210 to 225 | 231 to 300; degree 32 210 to 181 | 210 to 184 | 210 to 186 | 224 to
+//   229; degree 96 208 to 183 | 207 to 196 | 212 to 234 | 232 to 309; eight queries,
+//   degree 96 352 to 320 | 355 to 413 | 371 to 408 | 408 to 451
+//   fifteen queries (480 branches), 768 fp16, degree 64: 678 to 619 | 650 to 607 |
+//   681 to 693 | 735 to 816
+bool advance_eager(const AdvArgs& a, int team, int x_dtype, int block) {
     constexpr int64_t kMost = 96 << 10;
     const int64_t step = (int64_t)a.D * a.dim * (x_dtype == SWANN_DTYPE_F16 ? 2 : 4);
-    return block == 1024 && !a.codes && a.H == 1 && a.Hc > 0 && a.ts == 0 && step <= kMost;
+    return block == 1024 && !a.codes && a.H == 1 && a.Hc > 0 && a.ts == 0 &&
+           (int64_t)a.D * team <= block && step <= kMost;
 }
 
 template <typename XT>
@@ -1350,7 +1362,7 @@ void launch_eager(const AdvArgs& a, int team, size_t lds, hipStream_t st) {
 // fell from 0.79 to 0.72 and 0.53), so the blocks keep their dispatch order
 // instead, which spreads a query's branches over the XCDs; the table's and
 // bound's atomics are agent scope and stay coherent across XCDs.
-bool remap_branches(int J, int team, int x_dtype, int block, size_t lds, bool codes) {
+bool remap_branches(int J, int team, int x_dtype, int block, size_t lds, bool codes, bool eager) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
@@ -1360,16 +1372,16 @@ bool remap_branches(int J, int team, int x_dtype, int block, size_t lds, bool co
     int per_cu = 0;
     const bool f32 = x_dtype == SWANN_DTYPE_F32;
     switch (team) {
-        case 4: per_cu = f32 ? advance_occupancy<4, float>(block, lds, codes)
-                             : advance_occupancy<4, _Float16>(block, lds, codes); break;
-        case 8: per_cu = f32 ? advance_occupancy<8, float>(block, lds, codes)
-                             : advance_occupancy<8, _Float16>(block, lds, codes); break;
-        case 16: per_cu = f32 ? advance_occupancy<16, float>(block, lds, codes)
-                              : advance_occupancy<16, _Float16>(block, lds, codes); break;
-        case 32: per_cu = f32 ? advance_occupancy<32, float>(block, lds, codes)
-                              : advance_occupancy<32, _Float16>(block, lds, codes); break;
-        default: per_cu = f32 ? advance_occupancy<64, float>(block, lds, codes)
-                              : advance_occupancy<64, _Float16>(block, lds, codes); break;
+        case 4: per_cu = f32 ? advance_occupancy<4, float>(block, lds, codes, eager)
+                             : advance_occupancy<4, _Float16>(block, lds, codes, eager); break;
+        case 8: per_cu = f32 ? advance_occupancy<8, float>(block, lds, codes, eager)
+                             : advance_occupancy<8, _Float16>(block, lds, codes, eager); break;
+        case 16: per_cu = f32 ? advance_occupancy<16, float>(block, lds, codes, eager)
+                              : advance_occupancy<16, _Float16>(block, lds, codes, eager); break;
+        case 32: per_cu = f32 ? advance_occupancy<32, float>(block, lds, codes, eager)
+                              : advance_occupancy<32, _Float16>(block, lds, codes, eager); break;
+        default: per_cu = f32 ? advance_occupancy<64, float>(block, lds, codes, eager)
+                              : advance_occupancy<64, _Float16>(block, lds, codes, eager); break;
     }
     if (per_cu <= 0) (void)hipGetLastError();
     // Grouped only while a query's branches take at most a quarter of the
@@ -1515,8 +1527,9 @@ int swann_advance(const void* X, int x_dtype, int64_t n, int dim, const int32_t*
               code_margin};
     const int block = search_block_for(nb);
     const size_t lds = advance_lds(dim, D, L, codes != nullptr);
-    a.remap = remap_branches(J, team_size, x_dtype, block, lds, codes != nullptr) ? 1 : 0;
-    if (advance_eager(a, x_dtype, block)) {
+    const bool eager = advance_eager(a, team_size, x_dtype, block);
+    a.remap = remap_branches(J, team_size, x_dtype, block, lds, codes != nullptr, eager) ? 1 : 0;
+    if (eager) {
         if (x_dtype == SWANN_DTYPE_F32) launch_eager<float>(a, team_size, lds, (hipStream_t)stream);
         else launch_eager<_Float16>(a, team_size, lds, (hipStream_t)stream);
     } else if (codes)
