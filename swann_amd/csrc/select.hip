@@ -96,9 +96,8 @@ __global__ __launch_bounds__(256) void row_norms(const float* __restrict__ A, in
 // 2,000 x 131,072 x 1,024: 4.3 ms, 125 TFLOP/s (64 x 64 tiles on the vector
 // unit: 15.3 ms); 500 x 4,096 x 960: 50 against 162 us; 4,096 x 4,096 x 1,536:
 // 0.49 against 1.50 ms.
-// T = 128 reads each operand half as often from L2 as T = 64, and is taken once
-// its tiles give every CU two workgroups; below that the smaller tiles keep
-// more of the chip busy.
+// T = 128 reads each operand half as often from L2 as T = 64; the smaller tiles keep
+// more of the chip busy and pad a batch to fewer rows (gemm_run).
 // The vector path of the loads (VEC) needs rows of whole 16-byte chunks on a
 // 16-byte boundary; otherwise element loads fill the same stages.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -927,8 +926,13 @@ static int gemv_run(const float* Q, int64_t nq, int dim, const float* Vp, int64_
     return launch_status("select gemv");
 }
 
-// The distance matrix of a larger batch: 64 x 64 tiles, K split when the
-// tiles alone would not fill the chip.
+// The distance matrix of a larger batch, K split when the tiles alone would not fill
+// the chip.  128 x 128 tiles once they give every CU two workgroups, where they
+// multiply at most a sixteenth more rows of padding than 64 x 64 tiles do and the
+// rows allow 16-byte loads.  Whole selections, 128 to 64 tiles in ms, against 400,003
+// x 768: 9 queries 0.78 to 0.46, 64 0.83 to 0.51, 100 0.853 to 0.855, 160 1.51 to
+// 1.20, 256 1.59 to 1.61, 500 2.91 to 2.99, 1,000 5.51 to 5.84; element loads (131,072
+// x 99): 64 0.177 to 0.130, 256 0.303 to 0.263, 1,000 0.90 to 0.71.
 static int gemm_run(const float* Q, int64_t nq, int dim, const float* Vp, int64_t P, int metric,
                     const float* qn, float* vn, float* Dm, hipStream_t st) {
     if (metric == SWANN_METRIC_L2)
@@ -945,13 +949,12 @@ static int gemm_run(const float* Q, int64_t nq, int dim, const float* Vp, int64_
     float* out = Dm;
     if (S > 1) out = (float*)((char*)vn + ((P * 4 + 255) / 256) * 256);
     else kper = dim;
-    // 128 x 128 tiles once they give every CU two workgroups
     const bool vec = dim % 4 == 0 && (uintptr_t)Q % 16 == 0 && (uintptr_t)Vp % 16 == 0;
-    const bool big = ((P + 127) / 128) * ((nq + 127) / 128) >= 512;
+    const int64_t b64 = (nq + 63) / 64, b128 = (nq + 127) / 128;
+    const bool big = vec && ((P + 127) / 128) * b128 >= 512 && 32 * b128 <= 17 * b64;
     const int T = big ? 128 : 64;
     const dim3 grid((unsigned)(((P + T - 1) / T) * ((nq + T - 1) / T)), 1, (unsigned)S);
-    auto* kernel = big ? (vec ? dist_gemm<128, true> : dist_gemm<128, false>)
-                       : (vec ? dist_gemm<64, true> : dist_gemm<64, false>);
+    auto* kernel = big ? dist_gemm<128, true> : vec ? dist_gemm<64, true> : dist_gemm<64, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, Q, Vp, nq, P, dim, metric, qn, vn, out,
                        kper);
     if (S > 1)

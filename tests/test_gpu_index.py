@@ -1195,3 +1195,12 @@ def test_sweep_of_small_corpora(n, d, C, dtype):
         assert torch.equal(gd > 1e38, self_)
         assert ((gd.double() - want)[~self_].abs() <= bound).all()
         assert ((D.gather(1, gi.long()) - want)[~self_].abs() <= 2 * bound).all()
+
+
+@pytest.mark.parametrize("nq,P,d", [(64, 65536, 8), (65, 65536, 8), (129, 33000, 12),
+                                    (192, 33000, 12), (193, 33000, 12), (193, 33000, 13)])
+@pytest.mark.parametrize("metric", [0, 1])
+def test_selection_distances_where_the_tiles_change(nq, P, d, metric):
+    """Batches on both sides of the padding that chooses the tiles' size, and a width
+    without 16-byte loads."""
+    test_selection_distances_are_fp32_sums(nq, P, d, metric)
