@@ -855,12 +855,13 @@ __global__ __launch_bounds__(kStBlock, 4) void row_topk_join(float* __restrict__
 }
 
 // Parts a row of the streaming top-E is read in: enough workgroups for a few
-// on every CU, none shorter than 16,384 columns (eight steps) or 4 E.
-int topk_parts(int64_t nq, int64_t N, int E) {
-    const int64_t shortest = 4 * (int64_t)E > 16384 ? 4 * (int64_t)E : 16384;
+// on every CU, none shorter than 16,384 columns (eight steps).
+constexpr int kShortPart = 16384;
+static_assert(kShortPart >= 4 * (kTopBuf / 2), "a part holds its E best and their indices");
+int topk_parts(int64_t nq, int64_t N) {
     int64_t p = (1536 + nq - 1) / nq;
     if (nq >= 512) p = 1;
-    if (p > N / shortest) p = N / shortest;
+    if (p > N / kShortPart) p = N / kShortPart;
     return (int)(p < 1 ? 1 : p > 64 ? 64 : p);
 }
 
@@ -991,7 +992,7 @@ static int select_run(const float* Q, int64_t nq, int dim, const float* Vp, int6
         hipLaunchKernelGGL(row_topk_radix, dim3((unsigned)nq), dim3(kRadBlock), 0, st, Dm, P, E,
                            out_idx, out_dist);
     else {
-        const int parts = topk_parts(nq, P, E);
+        const int parts = topk_parts(nq, P);
         hipLaunchKernelGGL(row_topk_stream, dim3((unsigned)(nq * parts)), dim3(kStBlock), 0, st,
                            Dm, P, E, parts, out_idx, out_dist);
         if (parts > 1)

@@ -419,28 +419,21 @@ template <int METRIC, bool SHARE = false>
 __device__ __forceinline__ void append_own(const f32x16& v, int rbase, int64_t r0, int64_t c,
                                            float cn, float sc, const float* rs, const float* thr,
                                            const float* rnorm, int* cnt, const MfmaSweepArgs& a,
-                                           int split, int nterm_scale, const f32x16* vx,
-                                           int* needf, bool cok = true, bool shared = false,
-                                           bool fstage = false, int cl = 0, int* qn = nullptr,
-                                           int2* qe = nullptr) {
+                                           int split, int scaled, int* needf, bool cok = true,
+                                           bool shared = false, bool fstage = false, int cl = 0,
+                                           int* qn = nullptr, int2* qe = nullptr) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const float4 t4 = *reinterpret_cast<const float4*>(thr + rbase + g * 8);
         const float4 r4 = METRIC == SWANN_METRIC_L2
                               ? *reinterpret_cast<const float4*>(rnorm + rbase + g * 8)
                               : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 s4 = nterm_scale ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
-                                      : make_float4(1.f, 1.f, 1.f, 1.f);
+        const float4 s4 = scaled ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
+                                 : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int e = g * 4 + q;
-            float dot;
-            if (nterm_scale == 1)
-                dot = s4[q] * sc * (v[e] + (*vx)[e] * (1.0f / 2048.0f));
-            else if (nterm_scale == 2)
-                dot = s4[q] * v[e] * sc;
-            else
-                dot = v[e];
+            const float dot = scaled ? s4[q] * v[e] * sc : v[e];
             if (!cok) continue;
             const float d = dist_formula<METRIC>(dot, METRIC == SWANN_METRIC_L2 ? r4[q] : 0.f, cn);
             if (!(d < t4[q])) continue;
@@ -463,57 +456,32 @@ template <int METRIC>
 __device__ __forceinline__ void epilogue_block(const f32x16& v, int rbase, int64_t r0, int64_t c,
                                                bool cok, float cn, float sc, const float* rs,
                                                const float* thr, const float* rnorm, int* cnt,
-                                               const MfmaSweepArgs& a, int split, int nterm_scale,
-                                               const f32x16* vx, int* needf = nullptr,
-                                               const float* sthr = nullptr) {
+                                               const MfmaSweepArgs& a, int split, int scaled) {
     auto dist = [&](int e, const float4& r4, const float4& s4) {
         const int q = e & 3;
-        float dot;
-        if (nterm_scale == 1)
-            dot = s4[q] * sc * (v[e] + (*vx)[e] * (1.0f / 2048.0f));
-        else if (nterm_scale == 2)
-            dot = s4[q] * v[e] * sc;
-        else
-            dot = v[e];
+        const float dot = scaled ? s4[q] * v[e] * sc : v[e];
         return dist_formula<METRIC>(dot, METRIC == SWANN_METRIC_L2 ? r4[q] : 0.f, cn);
     };
     auto group = [&](int g, float4& t4, float4& r4, float4& s4) {
         t4 = *reinterpret_cast<const float4*>(thr + rbase + g * 8);
         r4 = METRIC == SWANN_METRIC_L2 ? *reinterpret_cast<const float4*>(rnorm + rbase + g * 8)
                                        : make_float4(0.f, 0.f, 0.f, 0.f);
-        s4 = nterm_scale ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
-                         : make_float4(1.f, 1.f, 1.f, 1.f);
+        s4 = scaled ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
+                    : make_float4(1.f, 1.f, 1.f, 1.f);
     };
     bool any = false;
-    if (sthr && nterm_scale != 1) {
-        // one compare per score against the row's screen threshold
-        const float ch = METRIC == SWANN_METRIC_L2 ? 0.5f * (cn - 1e-5f * fabsf(cn)) : 0.f;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const float4 h4 = *reinterpret_cast<const float4*>(sthr + rbase + g * 8);
-            const float4 s4 = nterm_scale ? *reinterpret_cast<const float4*>(rs + rbase + g * 8)
-                                          : make_float4(1.f, 1.f, 1.f, 1.f);
+    for (int g = 0; g < 4; ++g) {
+        float4 t4, r4, s4;
+        group(g, t4, r4, s4);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float dot = nterm_scale ? s4[q] * v[g * 4 + q] * sc : v[g * 4 + q];
-                any = any || (METRIC == SWANN_METRIC_IP ? dot > h4[q] : dot > ch + h4[q]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float4 t4, r4, s4;
-            group(g, t4, r4, s4);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) any = any || (dist(g * 4 + q, r4, s4) < t4[q]);
-        }
+        for (int q = 0; q < 4; ++q) any = any || (dist(g * 4 + q, r4, s4) < t4[q]);
     }
     any = any && cok;
     if (__ballot(any) == 0ull) return;
     asm volatile("" ::: "memory");           // rare path: reload rather than keep live
     if (!any) return;
-    append_own<METRIC>(v, rbase, r0, c, cn, sc, rs, thr, rnorm, cnt, a, split, nterm_scale, vx,
-                       needf);
+    append_own<METRIC>(v, rbase, r0, c, cn, sc, rs, thr, rnorm, cnt, a, split, scaled, nullptr);
 }
 
 // The foreign half of a tile's epilogue in the symmetric sweep: the same 32 x
@@ -617,7 +585,7 @@ __device__ __forceinline__ void self_out(f32x16& v, int rbase, int ccol) {
 }
 
 // ---------------------------------------------------------------------------
-// fp16 operands (NTERM = 1): workgroup tile 256 x 256 with eight waves of
+// The register-staged kernel: workgroup tile 256 x 256 with eight waves of
 // 128 x 64 (4 x 2 blocks of 32 x 32; 128 accumulators each), so two waves share
 // a SIMD and one's epilogue or wait overlaps the other's MFMAs.  K tile 32.  The
 // workgroup's work is one stream of (column tile, K tile) steps: global loads
@@ -663,7 +631,7 @@ __global__ __launch_bounds__(512, 1) void sweep_mfma256_kernel(MfmaSweepArgs a) 
         av[m] = r0 + lrow[m] < n;
         aoff[m] = (av[m] ? r0 + lrow[m] : n - 1) * (int64_t)dim + lpart[m];
     }
-    const int nk = (dim + kBK - 1) / kBK;
+    const int nk = dim / kBK;              // the plane's rows are whole K stages
     const int64_t nct = (n + kBN2 - 1) / kBN2;
     const int64_t nsteps = nct * nk;
 
@@ -671,18 +639,15 @@ __global__ __launch_bounds__(512, 1) void sweep_mfma256_kernel(MfmaSweepArgs a) 
         const f16x8 z = {};
         if (t >= nsteps) return;
         const int k0 = kt * kBK;
-        const bool kfull = k0 + kBK <= dim;
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
             const int64_t rb = cb + lrow[m];
             const bool bv = rb < n;
-            const bool kin = kfull || (k0 + lpart[m] < dim);
             const int64_t boff = (bv ? rb : n - 1) * (int64_t)dim + lpart[m];
-            const int kk = kin ? k0 : 0;                // never read past a row
-            const f16x8 va = *reinterpret_cast<const f16x8*>(a.hi + aoff[m] + kk);
-            const f16x8 vb = *reinterpret_cast<const f16x8*>(a.hi + boff + kk);
-            S.a[m] = (av[m] && kin) ? va : z;
-            S.b[m] = (bv && kin) ? vb : z;
+            const f16x8 va = *reinterpret_cast<const f16x8*>(a.hi + aoff[m] + k0);
+            const f16x8 vb = *reinterpret_cast<const f16x8*>(a.hi + boff + k0);
+            S.a[m] = av[m] ? va : z;
+            S.b[m] = bv ? vb : z;
         }
     };
     auto lstore = [&](const Stage& S, int buf) {
@@ -766,7 +731,7 @@ __global__ __launch_bounds__(512, 1) void sweep_mfma256_kernel(MfmaSweepArgs a) 
                     asm volatile("" : "+v"(rbase));
                     if (diag) self_out(acc[i][j], rbase, wn * 64 + j * 32 + (lane & 31));
                     epilogue_block<METRIC>(acc[i][j], rbase, r0, c, cok, cn[j], cs[j], rscale,
-                                           thr, rnorm, cnt, a, 0, SCALED ? 2 : 0, nullptr);
+                                           thr, rnorm, cnt, a, 0, SCALED);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -1201,9 +1166,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
                     if (own & valid) {
                         asm volatile("" ::: "memory");   // rare path: reload, do not keep live
                         append_own<METRIC, true>(acc[i][j], rbase, r0, c, cn[j], cs[j], rscale,
-                                                 thr, rnorm, cnt, a, split, SCALED ? 2 : 0,
-                                                 nullptr, &need[tpar], cok, run[4] != 0, fstage,
-                                                 c - cb, &fqn, fq);
+                                                 thr, rnorm, cnt, a, split, SCALED, &need[tpar],
+                                                 cok, run[4] != 0, fstage, c - cb, &fqn, fq);
                     }
                     if (frn & valid) {
                         asm volatile("" ::: "memory");
