@@ -645,7 +645,7 @@ __global__ __launch_bounds__(512, 1) void sweep_mfma256_kernel(MfmaSweepArgs a) 
             const bool bv = rb < n;
             const int64_t boff = (bv ? rb : n - 1) * (int64_t)dim + lpart[m];
             const f16x8 va = *reinterpret_cast<const f16x8*>(a.hi + aoff[m] + k0);
-            const f16x8 vb = *reinterpret_cast<const f16x8*>(a.hi + boff + k0);
+            const f16x8 vb = *reinterpret_cast<const f16x8*>(a.cols + boff + k0);
             S.a[m] = av[m] ? va : z;
             S.b[m] = bv ? vb : z;
         }
@@ -2486,7 +2486,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
     *used = 1;
     // the direct loads address a stage's 256 rows with 32-bit byte offsets
     const bool off32 = (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32);
-    if ((uintptr_t)hi % 16 == 0 && off32 && (split3 || !option_on(kOptSweepRegstage))) {
+    if ((uintptr_t)hi % 16 == 0 && off32 && !option_on(kOptSweepRegstage)) {
         const int64_t ntile = (n + kBM2 - 1) / kBM2;
         const bool orders = sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed);
         if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !(orders && capturing(st))) {

@@ -1204,3 +1204,25 @@ def test_selection_distances_where_the_tiles_change(nq, P, d, metric):
     """Batches on both sides of the padding that chooses the tiles' size, and a width
     without 16-byte loads."""
     test_selection_distances_are_fp32_sums(nq, P, d, metric)
+
+
+@pytest.mark.parametrize("d", [96, 100])
+@pytest.mark.parametrize("how", ["off 16 bytes", "sweep_regstage"])
+def test_register_staged_sweep_reads_the_column_plane(opt, d, how):
+    """A workspace off a 16-byte boundary (and the option) takes the register-staged
+    kernel, which at three parts a row reads two planes: the same lists."""
+    from swann_amd import _lib
+    n, C = 1500, 48
+    X = torch.from_numpy(gaussian(n, d, d, False)).cuda()
+    wi, wd = B.knn_candidates(X, C, metric="l2")
+    off = 4 if how == "off 16 bytes" else 0
+    if not off:
+        opt(sweep_regstage=1)
+    need = int(_lib.lib().swann_sweep_workspace_size(n, d, 0, C))
+    ws = torch.empty(need + 16, dtype=torch.uint8, device="cuda")
+    gi = torch.empty((n, C), dtype=torch.int32, device="cuda")
+    gd = torch.empty((n, C), device="cuda")
+    _lib.call("swann_build_sweep", _lib.ptr(X), 0, n, d, 1, C, _lib.ptr(gi), _lib.ptr(gd),
+              _lib.ptr(ws[off:]), _lib.stream_of(X.device))
+    assert torch.allclose(gd, wd, rtol=1e-5, atol=0)
+    assert (gi != wi).float().mean() < 1e-3
