@@ -251,11 +251,21 @@ int swann_select_nearest_noalloc(const float* Q, int64_t nq, int dim, const floa
  *
  * Sweep (build.py:28-43): exact top-C neighbours of every row, self
  * excluded (3.4e38), ascending, as (cand [n, C] int32, cdist [n, C] fp32) with
- * IP: 1 - <a,b>; L2: max(0, |b|^2 - 2<a,b> + |a|^2).  When dim % 8 == 0 the
- * scores come from fp16 MFMA tiles (fp16 corpus: exact products; fp32 corpus:
- * a power-of-two row-scaled fp16 screen keeps C+32 per row, which are then
- * re-ranked with exact fp32 dot products); otherwise from fp32 SIMT tiles.
- * `workspace`: swann_sweep_workspace_size bytes.
+ * IP: 1 - <a,b>; L2: max(0, |b|^2 - 2<a,b> + |a|^2).  The scores come from fp16
+ * MFMA tiles, of rows padded to a multiple of 64 where they are not one:
+ *   fp16 corpus: exact products, fp32 sums;
+ *   fp32 corpus, dim % 8 == 0: an fp16 screen (scaled by a power of two a row
+ *     where the values need it) keeps C+32 per row, which are then re-ranked with
+ *     exact fp32 dot products;
+ *   fp32 corpus, dim % 8 != 0, 64 <= dim <= 16384: the same with rows in three fp16
+ *     parts, each factor to 2^-22, so that the rows kept are chosen about as fp32
+ *     sums choose them (at most the list limit: C > 224 leaves the re-rank less
+ *     than 32 entries of slack);
+ * or from fp32 SIMT tiles: fp32 rows of any other width that is no multiple of 8, and
+ * corpora of a few hundred rows of small ragged widths.
+ * `workspace`: swann_sweep_workspace_size bytes: per row one or more candidate
+ * lists and, where the corpus is not its own plane, one fp16 copy (two at three
+ * parts a row: 12 bytes an element).
  * The call waits for the GPU (small read-backs) where it must choose: for an fp32
  * corpus with dim % 8 == 0 (the rows' range), and from 192 row panels of 256 unless
  * fp32 rows are no multiple of 8 (the clustering, the locality order, the repair).

@@ -1219,8 +1219,10 @@ int prune_run(const void* X, int x_dtype, int64_t n, int dim, int metric, const 
               const uint8_t* protect, int32_t* out, const int32_t* order, float* rscale,
               hipStream_t st) {
     // the Gram on MFMA (option prune_simt: on SIMT): 16-byte loads where the
-    // rows are whole aligned chunks, element loads otherwise (20,011 rows of 100
-    // fp32, C = 64: 1.04 ms, on SIMT 1.35)
+    // rows are whole aligned chunks, element loads otherwise.  SIMT to MFMA, C = 128,
+    // ms: 20,000 x 100 fp32 (16-byte loads) 1.87 to 1.27; element loads 20,000 x 99
+    // 1.86 to 1.51 (fp16 1.74 to 1.32), 20,000 x 201 2.74 to 2.26 (2.71 to 1.63),
+    // 10,000 x 1,001 5.06 to 3.05 (5.10 to 1.81)
     const bool simt = option_on(kOptPruneSimt);
     const bool f32 = x_dtype == SWANN_DTYPE_F32;
     const bool vec = dim % (f32 ? 4 : 8) == 0 && (uintptr_t)X % 16 == 0;

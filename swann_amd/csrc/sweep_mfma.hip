@@ -9,7 +9,9 @@
 //   * an fp32 corpus is screened: rows are scaled by a power of two s and
 //     rounded once to fp16, s_a s_b (h_a . h_b) ranks the candidates to within
 //     ~1e-4 relative, the sweep keeps C + 32 per row, and the caller re-ranks
-//     those in fp32 (one gather of C + 32 rows per row, not a second sweep).
+//     those in fp32 (one gather of C + 32 rows per row, not a second sweep);
+//     rows that are no multiple of 8 go in three parts (split3_rows), each factor
+//     to 2^-22.
 // Epilogue per tile: score -> distance by the reference formula, test against
 // the row's running threshold (LDS), append survivors to the row's buffer;
 // rows near capacity are compacted to their C best (wave-level exact select).
@@ -2379,8 +2381,8 @@ inline bool sweep_sym(int64_t ntile) {
 }
 
 // Whether the symmetric sweep looks for clusters and, where the rows form some,
-// runs in the locality order: by default from 192 row panels (n > 48,896), whenever
-// sweep_sym = 1 forces the symmetric sweep.  Order, bounds and their read-backs cost
+// runs in the locality order: by default from 192 row panels (n > 48,896), and
+// whenever sweep_sym = 1 forces the symmetric sweep.  Order, bounds and their read-backs cost
 // about 2 ms however few the tiles left.  Gaussian mixtures of 8 to n / 700 clusters,
 // C = 128, ordered against the circle in the rows' order, in ms (fp16 768 wide; fp16
 // 128; fp32 1,536): 8,000 rows 1.87 to 2.14 against 0.86 (one-sided 1.12); 24,000

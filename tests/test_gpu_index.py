@@ -316,7 +316,7 @@ def test_mfma_sweep_other_layouts_match_oracle(opt, switch, metric, dtype):
     both of its panels' rows, in bands of launches), all chosen by
     environment at each call, keep the oracle's lists like the default
     layout; so does the symmetric sweep whose second lists are made to
-    overflow (4 entries of room), which must redo the sweep one-sided, and an
+    overflow (4 entries of room), whose panels are swept again one-sided, and an
     fp32 corpus screened on a row-scaled fp16 plane (the default takes these
     corpora's values into fp16 unscaled).  Each is an option of the library
     (swann_set_option), set for the test."""
@@ -634,7 +634,7 @@ def test_index_capture_matches_eager_search():
 def test_select_small_and_large_batches_match_oracle(nq, metric):
     """Selection at every batch shape: the one-pass product for batches of up
     to 8 (16-byte loads, and element loads at d = 70), split-K partials for
-    small grids, the radix top-E for rows up to 16384 and the chunked bitonic
+    small grids, the radix top-E for rows up to 16384 and the streamed one
     beyond; ties (duplicated catalogue rows) resolve to the lower index, as the oracle's
     (d, index) order.  With two or more queries, query 1 is NaN throughout:
     its distances cannot be ranked, so its E entries come in no stated order,
@@ -976,7 +976,8 @@ def test_fp16_sweep_under_graph_capture():
 @pytest.mark.parametrize("metric", ["ip", "l2"])
 def test_sweep_and_prune_at_any_width(n, d, dtype, C, metric):
     """Widths that are no whole K stage of the tiles (the corpus copied to a padded
-    plane, or split in three parts where fp32 rows are no multiple of 8) and rows
+    plane, split in three parts where fp32 rows of 64 or more are no multiple of 8, or
+    on the SIMT tiles) and rows
     off a 16-byte boundary (the prune's element loads): distances within fp32
     rounding of the float64 top-C, the prune's rows the SIMT Gram's."""
     from swann_amd import _lib
