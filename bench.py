@@ -65,7 +65,7 @@ MFMA_F16_PEAK = 2.5e15              # dense fp16/bf16 MFMA, MI355X
 # claims layout (Index._claims: "bits<n>" or the table's slots); otherwise `traffic`
 # is reported as null.
 PMC_TRAFFIC = {
-    ("c3", 1_000_000, 10_000, 64, 44, 64, 0.3, "bits1048576", "5527c75807f6f5f0"): 4.860e12,
+    ("c3", 1_000_000, 10_000, 64, 44, 64, 0.3, "bits1048576", "4bdfb8df2bef72f1"): 4.860e12,
 }
 
 
