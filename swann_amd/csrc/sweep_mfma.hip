@@ -100,15 +100,19 @@ __global__ __launch_bounds__(256) void split_rows(const float* __restrict__ X, i
 // it meets the other row's hi and is infinite with that one's sign, as the fp32
 // product is; so a nonzero y's hi is never zero (at least 2^-24, which lo then
 // takes back), and the row's scale is that of its finite elements.
+// With `perm` the planes' row r (and its scale and normp) is the corpus's perm[r].
 __global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, int64_t n, int dim,
-                                                   int k8, int ld, _Float16* __restrict__ pa,
+                                                   int k8, int ld, const int* __restrict__ perm,
+                                                   _Float16* __restrict__ pa,
                                                    _Float16* __restrict__ pb,
                                                    float* __restrict__ scale,
-                                                   float* __restrict__ norm) {
+                                                   float* __restrict__ norm,
+                                                   float* __restrict__ normp) {
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (r >= n) return;
-    const float* x = X + r * dim;
+    const int64_t rx = perm ? perm[r] : r;
+    const float* x = X + rx * dim;
     float m = 0.f, s2 = 0.f;
     for (int t = lane; t < dim; t += 64) {
         const float v = x[t];
@@ -136,7 +140,11 @@ __global__ __launch_bounds__(256) void split3_rows(const float* __restrict__ X, 
         pa[r * ld + t] = part == 0 ? h : !fin ? z : part == 2 ? l : h;
         pb[r * ld + t] = part == 0 ? h : !fin ? z : part == 1 ? l : h;
     }
-    if (lane == 0) { scale[r] = s; norm[r] = s2; }
+    if (lane == 0) {
+        scale[r] = s;
+        norm[rx] = s2;
+        if (normp) normp[r] = s2;
+    }
 }
 
 // fp16 rows copied to a plane `ld` wide, zero past dim.
@@ -252,7 +260,6 @@ struct MfmaSweepArgs {
     int sym;
     int64_t b0, b1;
     const float* gthr;           // [n] a row's threshold when the launch began
-    int* ovf;                    // foreign appends that found no room
     int fcap;                    // room in list 1 (<= cap; smaller only as a test hook)
     // one-sided sweep of listed row panels only (the repair of rows whose
     // second list overflowed): workgroup g takes panel plist[g / G]
@@ -395,12 +402,10 @@ __device__ __forceinline__ void push_second(const MfmaSweepArgs& a, bool fstage,
         return;
     }
     const int p = atomicAdd(&a.bcnt[row * 2 + 1], 1);
-    if (p < a.fcap) {
+    if (p < a.fcap) {                    // past it the merge sees the count
         const int64_t o = (row * 2 + 1) * (int64_t)a.cap + p;
         a.bkey[o] = d;
         a.bid[o] = (int32_t)id;
-    } else {
-        atomicAdd(a.ovf, 1);
     }
 }
 
@@ -1054,8 +1059,6 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
                     const int64_t o = ((int64_t)w.row * 2 + 1) * (int64_t)a.cap + fslot;
                     a.bkey[o] = __int_as_float(e.y);
                     a.bid[o] = (int32_t)w.id;
-                } else {
-                    atomicAdd(a.ovf, 1);
                 }
             }
             if (tid == 0) fqn = 0;      // the next refill is after the next barrier
@@ -1196,8 +1199,6 @@ __global__ __launch_bounds__(WAVES * 64, 1) void sweep_dma_kernel(MfmaSweepArgs 
                 const int64_t o = ((int64_t)w.row * 2 + 1) * (int64_t)a.cap + p;
                 a.bkey[o] = __int_as_float(e.y);
                 a.bid[o] = (int32_t)w.id;
-            } else {
-                atomicAdd(a.ovf, 1);
             }
         }
     }
@@ -2181,7 +2182,13 @@ __global__ void pivot_place(const int* __restrict__ lab, int64_t n, int* pcur,
     if (r < n) perm[atomicAdd(&pcur[lab[r]], 1)] = (int)r;
 }
 
-// The ordered copy: row perm[i] of the plane, its norm and scale at i.
+// The circle's row order (spread_step): row p s mod n at p.
+__global__ void spread_rows(int* __restrict__ perm, int64_t n, int64_t s) {
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p < n) perm[p] = (int)(p * s % n);
+}
+
+// A reordered copy: row perm[i] of the plane, its norm and scale at i.
 __global__ __launch_bounds__(256) void gather_rows(const _Float16* __restrict__ h, int64_t n,
                                                    int dim, const int* __restrict__ perm,
                                                    const float* __restrict__ xn,
@@ -2408,6 +2415,27 @@ inline bool capturing(hipStream_t st) {
     return c != hipStreamCaptureStatusNone;
 }
 
+// Around the circle the rows are not swept in their own order but p s mod n at p, s
+// about 0.618 n and prime to n, so that every panel is an even sample of the corpus.
+// A launch's second lists hold what beats the thresholds the last merge left, and
+// those are only as good as the panels seen: in an order the distances follow (rows
+// sorted by norm, along a line, by cluster) the panels seen say little of the next
+// ones, nearly all of which then beat them, and every list overflows and is swept
+// again.  C = 128, own order and spread (one-sided), ms: rows by rising norm, l2,
+// 8,000 x 768 fp16 4.93 and 0.74 (0.98), 60,000 134.6 and 6.5 (10.7), 60,000 x 100
+// fp32 97.1 and 7.3 (27.6); along a line, ip, 20,000 x 64 fp16 21.3 and 1.4 (5.4).
+// Rows in no order pay for the copy: 60,000 x 768 fp16 7.03 to 7.10, 100,000 x 1,536
+// 24.61 to 24.66; rows stored by cluster lose what their own order gave (20,000 x 768,
+// 50 clusters 0.86 to 1.88, one-sided 4.47).
+inline int64_t spread_step(int64_t n) {
+    int64_t s = (int64_t)(0.6180339887498949 * (double)n);
+    for (s = s < 1 ? 1 : s;; ++s) {
+        int64_t a = s, b = n;
+        while (b) { const int64_t t = a % b; a = b; b = t; }
+        if (a == 1) return s;
+    }
+}
+
 // Waves per direct-load workgroup: 16 (64 x 64 wave tiles, the default) or
 // 8 (128 x 64; option sweep_waves).
 inline int sweep_waves() { return option(kOptSweepWaves) == 8 ? 8 : 16; }
@@ -2428,9 +2456,28 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
     const bool split3 = plane_split3(xdim, x_dtype);
     g_tiles_scored = 0;
     g_dense_panels = 0;
-    const int64_t ntile_all = (n + kBM2 - 1) / kBM2;
+    const int64_t ntile = (n + kBM2 - 1) / kBM2;
+    const unsigned nb256 = (unsigned)((n + 255) / 256);
+    // the direct loads read whole 16-byte chunks of a plane and address a stage's 256
+    // rows with 32-bit byte offsets
+    const bool own = x_dtype == SWANN_DTYPE_F16 && dim == xdim;
+    const bool direct = (uintptr_t)(own ? X : extra) % 16 == 0 &&
+                        (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32) &&
+                        !option_on(kOptSweepRegstage);
+    const bool orders = sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed);
+    const bool symmetric = direct && (uintptr_t)extra % 16 == 0 && splits >= 2 &&
+                           sweep_sym(ntile) && sweep_waves() == 16 && !(orders && capturing(st));
     float* xn = (float*)extra; extra += al256(n * 4);
     float* scale = (float*)extra; extra += al256(n * 4);
+    // the circle's order, and the norms in it (a sweep that may order the rows
+    // carves them with the rest of that)
+    int* perm = nullptr;
+    float* xnp = nullptr;
+    if (symmetric && !orders) {
+        perm = (int*)extra; extra += al256(n * 4);
+        xnp = (float*)extra; extra += al256(n * 4);
+        hipLaunchKernelGGL(spread_rows, dim3(nb256), dim3(256), 0, st, perm, n, spread_step(n));
+    }
     const _Float16* hi;
     const _Float16* cols = nullptr;      // the column panels' plane, where it is another
     int scaled = x_dtype == SWANN_DTYPE_F16 ? 0 : 1;
@@ -2451,7 +2498,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
         _Float16* hc = (_Float16*)extra;
         extra += al256(n * (int64_t)dim * 2);
         hipLaunchKernelGGL(split3_rows, dim3(nrb), dim3(256), 0, st, (const float*)X, n, xdim,
-                           (xdim + 7) / 8 * 8, dim, h, hc, scale, xn);
+                           (xdim + 7) / 8 * 8, dim, (const int*)perm, h, hc, scale, xn, xnp);
         hi = h;
         cols = hc;
     } else {
@@ -2482,16 +2529,12 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
         hi = h;
     }
     MfmaSweepArgs a{hi, cols ? cols : hi, scale, xn, n, dim, metric, C, cap, bkey, bid, bcnt, scaled, 1,
-                    0, 0, 0, nullptr, nullptr, cap};                 // the rest 0
-    const unsigned grid = (unsigned)((n + kBM2 - 1) / kBM2);
+                    0, 0, 0, nullptr, cap};                          // the rest 0
+    const unsigned grid = (unsigned)ntile;
     const bool ip = metric == SWANN_METRIC_IP;
     *used = 1;
-    // the direct loads address a stage's 256 rows with 32-bit byte offsets
-    const bool off32 = (int64_t)dim * 2 * kBM2 < (int64_t(1) << 32);
-    if ((uintptr_t)hi % 16 == 0 && off32 && !option_on(kOptSweepRegstage)) {
-        const int64_t ntile = (n + kBM2 - 1) / kBM2;
-        const bool orders = sweep_orders(ntile) && !split3 && !option_on(kOptSweepNoseed);
-        if (splits >= 2 && sweep_sym(ntile) && sweep_waves() == 16 && !(orders && capturing(st))) {
+    if (direct) {
+        if (symmetric) {
             // symmetric sweep: tile (I, J), J >= I, scored once for the rows of
             // both panels; launched in bands of J - I (1, 1, 2, 4, ... 256, then
             // kBandMax at a time) with a merge after each, so every launch
@@ -2505,7 +2548,6 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
             s.splits = 2;
             s.sym = 1;
             s.gthr = gthr;
-            s.ovf = ovf;
             s.mcnt = mcnt;
             s.fcap = cap;
             {                                       // option sweep_sym_fcap: force overflow
@@ -2580,7 +2622,6 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 }
                 return SWANN_OK;
             };
-            const unsigned nb256 = (unsigned)((n + 255) / 256);
             float* seed = nullptr;
             hipLaunchKernelGGL(fill_zero, dim3(nb256), dim3(256), 0, st, flag, (int)n);
             int* plist = nullptr;
@@ -2594,9 +2635,9 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 // the order's workspace (seed_bytes, repair_bytes)
                 float* sk = (float*)extra; extra += al256(n * kSketch * 4);
                 int* lab = (int*)extra; extra += al256(n * 4);
-                int* perm = (int*)extra; extra += al256(n * 4);
+                perm = (int*)extra; extra += al256(n * 4);
                 seed = (float*)extra; extra += al256(n * 4);
-                float* xnp = (float*)extra; extra += al256(n * 4);
+                xnp = (float*)extra; extra += al256(n * 4);
                 float* scp = (float*)extra; extra += al256(n * 4) * 2;
                 int* pcnt = (int*)extra; extra += al256(kMaxPivots * 4);
                 _Float16* hp = (_Float16*)extra; extra += al256(n * (int64_t)dim * 2);
@@ -2698,7 +2739,16 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                                        perm);
                 }
                 if (!clustered) {
-                    seed = nullptr;              // the rows' own order, no seeds
+                    // around the circle, no seeds
+                    seed = nullptr;
+                    hipLaunchKernelGGL(spread_rows, dim3(nb256), dim3(256), 0, st, perm, n,
+                                       spread_step(n));
+                    hipLaunchKernelGGL(gather_rows, dim3(nrb), dim3(256), 0, st, hi, n, dim, perm,
+                                       xn, scaled ? scale : nullptr, hp, xnp, scp);
+                    s.hi = s.cols = hp;
+                    s.xn = xnp;
+                    s.scale = scp;
+                    ordered = perm;
                     goto plain;
                 }
                 hipLaunchKernelGGL(gather_rows, dim3(nrb), dim3(256), 0, st, hi, n, dim, perm, xn,
@@ -2833,6 +2883,18 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                                        seed);
                 }
             }
+            else {
+                if (!split3) {
+                    float* scp = (float*)extra; extra += al256(n * 4);
+                    _Float16* hp = (_Float16*)extra; extra += al256(n * (int64_t)dim * 2);
+                    hipLaunchKernelGGL(gather_rows, dim3(nrb), dim3(256), 0, st, hi, n, dim, perm,
+                                       xn, scaled ? scale : nullptr, hp, xnp, scp);
+                    s.hi = s.cols = hp;
+                    s.scale = scp;
+                }
+                s.xn = xnp;
+                ordered = perm;
+            }
         plain:
             hipLaunchKernelGGL(sym_init, dim3(nb256), dim3(256), 0, st, gthr, bcnt, ovf, n,
                                (const float*)seed, mcnt);
@@ -2858,6 +2920,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
                 }
                 g_tiles_scored += host_tiles;
                 *used = 2;
+                *perm_out = ordered;
                 return launch_status("sweep (mfma, circle repair)");
             }
         swept:
@@ -3009,7 +3072,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
         }
         a.splits = splits;
         *used = splits;
-        g_tiles_scored += ntile_all * ntile_all;          // every tile, one-sided
+        g_tiles_scored += ntile * ntile;          // every tile, one-sided
         const unsigned grid = (unsigned)((n + kBM2 - 1) / kBM2 * splits);
         if (sweep_waves() == 16) {
             if (scaled) {
@@ -3028,7 +3091,7 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
         }
         return launch_status("sweep (mfma, direct loads)");
     }
-    g_tiles_scored += ntile_all * ntile_all;
+    g_tiles_scored += ntile * ntile;
     if (scaled) {
         if (ip) hipLaunchKernelGGL((sweep_mfma256_kernel<SWANN_METRIC_IP, 1>), dim3(grid), dim3(kT2), 0, st, a);
         else hipLaunchKernelGGL((sweep_mfma256_kernel<SWANN_METRIC_L2, 1>), dim3(grid), dim3(kT2), 0, st, a);
@@ -3039,23 +3102,24 @@ int sweep_mfma_run(const void* X, int x_dtype, int64_t n, int xdim, int metric, 
     return launch_status("sweep (mfma)");
 }
 
-// Extra workspace: norms, scales, the fp16 plane (an fp32
-// corpus, or an fp16 one of another width than the plane's), the
-// symmetric sweep's thresholds and overflow count, and its seed pre-pass.
+// Extra workspace: norms, scales, the fp16 plane (an fp32 corpus, or an fp16 one of
+// another width than the plane's), and where the sweep runs symmetric its thresholds,
+// counts and flags with either the circle's order and copy or, if it may order the
+// rows, that order's scratch (which the circle's fits; a superset of the run's
+// conditions, so the run never finds less than it needs: a corpus the clustering
+// check declines at run time, or option sweep_noseed, still reserves it).
 int64_t sweep_mfma_extra_bytes(int64_t n, int xdim, int x_dtype) {
     const int dim = plane_width(xdim, x_dtype);
-    const int64_t planes = plane_split3(xdim, x_dtype) ? 2
-                           : x_dtype == SWANN_DTYPE_F16 && dim == xdim ? 0 : 1;
-    const int64_t base = al256(n * 4) * 2 + planes * al256(n * (int64_t)dim * 2) +
-                         al256(n * 4) + 256 + al256(n * 4) * 2;
-    // the locality order, seeds and panel repair run only in the symmetric
-    // direct-load sweep past its seed bands; only a sweep that may take that
-    // path reserves their scratch (a superset of the run's conditions, so the
-    // run never finds less than it needs: a corpus the clustering check
-    // declines at run time, or option sweep_noseed, still reserves it)
+    const int64_t plane = al256(n * (int64_t)dim * 2);
+    const bool split3 = plane_split3(xdim, x_dtype);
+    const int64_t planes = split3 ? 2 : x_dtype == SWANN_DTYPE_F16 && dim == xdim ? 0 : 1;
+    int64_t b = al256(n * 4) * 2 + planes * plane;
     const int64_t ntile = (n + kBM2 - 1) / kBM2;
-    const bool seeded = !plane_split3(xdim, x_dtype) && sweep_sym(ntile) && sweep_orders(ntile);
-    return base + (seeded ? seed_bytes(n, dim) + repair_bytes(1024) : 0);   // cap <= 1024
+    if (!sweep_sym(ntile)) return b;
+    b += al256(n * 4) * 3 + 256;
+    if (sweep_orders(ntile) && !split3)
+        return b + seed_bytes(n, dim) + repair_bytes(1024);      // cap <= 1024
+    return b + al256(n * 4) * 2 + (split3 ? 0 : al256(n * 4) + plane);
 }
 
 // Column splits of the direct-load sweep: enough workgroups to give every

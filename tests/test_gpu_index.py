@@ -1227,3 +1227,25 @@ def test_register_staged_sweep_reads_the_column_plane(opt, d, how):
               _lib.ptr(ws[off:]), _lib.stream_of(X.device))
     assert torch.allclose(gd, wd, rtol=1e-5, atol=0)
     assert (gi != wi).float().mean() < 1e-3
+
+
+@pytest.mark.parametrize("n", [8500, 49200])
+@pytest.mark.parametrize("how,metric", [("up", "ip"), ("up", "l2"), ("down", "ip")])
+def test_rows_sorted_by_norm_overflow_no_list(opt, n, how, metric):
+    """Rows stored by their norm, which the distances follow: the circle takes them
+    spread over the panels, so no second list overflows (where the host repairs, as
+    sweep_sym = 1 has it, it would sweep panels again: the tiles are the circle's),
+    and the lists are the one-sided sweep's."""
+    from swann_amd import _lib
+    g = torch.Generator().manual_seed(n)
+    r = torch.linspace(0.2, 5, n)
+    X = torch.randn((n, 64), generator=g) / 8 * (r if how == "up" else r.flip(0))[:, None]
+    X = X.half().cuda()
+    nt = (n + 255) // 256
+    opt(sweep_sym=1)
+    gi, gd = B.knn_candidates(X, 64, metric=metric)
+    assert int(_lib.lib().swann_sweep_tiles_scored()) == nt * (nt + 1) // 2
+    opt(sweep_sym=0)
+    wi, wd = B.knn_candidates(X, 64, metric=metric)
+    assert torch.equal(gd, wd)
+    assert (gi != wi).float().mean() < 1e-3
