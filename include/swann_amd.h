@@ -264,10 +264,11 @@ int swann_select_nearest_noalloc(const float* Q, int64_t nq, int dim, const floa
  * or from fp32 SIMT tiles: fp32 rows of any other width that is no multiple of 8, and
  * corpora of a few hundred rows of small ragged widths.
  * `workspace`: swann_sweep_workspace_size bytes: per row one or more candidate
- * lists and, where the corpus is not its own plane, one fp16 copy (two at three
- * parts a row: 12 bytes an element).
+ * lists, where the corpus is not its own plane one fp16 copy (two at three parts a
+ * row: 12 bytes an element), and from 32 row panels a reordered copy (not at three
+ * parts).
  * The call waits for the GPU (small read-backs) where it must choose: for an fp32
- * corpus with dim % 8 == 0 (the rows' range), and from 192 row panels of 256 unless
+ * corpus with dim % 8 == 0 (the rows' range), and from 1,024 row panels of 256 unless
  * fp32 rows are no multiple of 8 (the clustering, the locality order, the repair).
  * Elsewhere it only launches.  Under stream capture a sweep that may order its
  * rows is recorded one-sided; an fp32 corpus with dim % 8 == 0 cannot be captured. */

@@ -2388,18 +2388,20 @@ inline bool sweep_sym(int64_t ntile) {
 }
 
 // Whether the symmetric sweep looks for clusters and, where the rows form some,
-// runs in the locality order: by default from 192 row panels (n > 48,896), and
-// whenever sweep_sym = 1 forces the symmetric sweep.  Order, bounds and their read-backs cost
-// about 2 ms however few the tiles left.  Gaussian mixtures of 8 to n / 700 clusters,
-// C = 128, ordered against the circle in the rows' order, in ms (fp16 768 wide; fp16
-// 128; fp32 1,536): 8,000 rows 1.87 to 2.14 against 0.86 (one-sided 1.12); 24,000
-// 2.7 to 2.9 against 2.2; 1.7 to 2.0 against 2.0; 5.8 to 6.5 against 4.4 to 5.0;
-// 40,000 3.2 to 3.9 against 4.1; 2.1 to 2.8 against 3.7; 7.6 to 9.6 against 8.0 to
-// 9.8; 49,200 3.4 to 4.4 against 5.6; 2.2 to 3.1 against 5.0; 8.2 to 11.6 against
-// 10.7 to 13.3; 200,000 8.6 to 18.9 against 56.  Rows stored cluster by cluster are
-// in a locality order already, which the check does not see: there the circle stays
-// ahead to 100,000 or so (60,000 x 768 fp16: 7.2 against 3.9, one-sided 14.3).
-constexpr int64_t kOrderPanels = 192;
+// runs in the locality order: by default from 1,024 row panels (n > 261,888), and
+// whenever sweep_sym = 1 forces the symmetric sweep.  Clean clusters gain much
+// earlier, but what the check takes for clusters need not bound the tiles, and then
+// the order costs its bounds, loose seeds and a repair of every panel.  C = 128,
+// ordered, around the circle and one-sided, in ms:
+//   mixture of 8 clusters, l2, 768 fp16: 8,000 rows 1.87, 0.86, 1.12; 24,000 2.9, 2.2,
+//   4.2; 49,200 4.4, 5.6, 11.7; 200,000 18.9, 56, 108
+//   16 clusters and 20% rows far from them, l2, 256 fp16: 49,200 rows 13.9, 4.4, 8.8;
+//   100,000 24.2, 11.8, 21.4; 200,000 69.1, 34.4, 63.4 (at 200 clusters 74.9, 34.3, 65.9)
+//   clusters whose norms spread by e, ip, 256 fp16: 49 of 49,200 rows 15.6, 4.2, 9.2;
+//   100 of 100,000 22.9, 11.0, 21.4
+// Below the line the circle takes about half of the one-sided sweep's time whatever
+// the rows, and reads nothing back.
+constexpr int64_t kOrderPanels = 1024;
 inline bool sweep_orders(int64_t ntile) {
     return ntile > 2 * kSeedBand && (ntile >= kOrderPanels || option(kOptSweepSym) == 1);
 }

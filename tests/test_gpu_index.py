@@ -1077,9 +1077,9 @@ def test_narrow_fp32_rows_are_ranked_by_fp32_sums(d):
     assert (kth - got).max() <= 4.01 * 2.0 ** -24 * float(S.max())
 
 
-@pytest.mark.parametrize("n,ordered", [(9000, False), (48896, False), (48897, True)])
+@pytest.mark.parametrize("n,ordered", [(9000, False), (261888, False), (261889, True)])
 def test_clustered_rows_are_ordered_only_where_it_pays(opt, n, ordered):
-    """A mixture of 8 clusters: below 192 row panels the sweep goes round the
+    """A mixture of 8 clusters: below 1,024 row panels the sweep goes round the
     circle, every tile once; from there it leaves out what the clusters' bounds
     show empty.  Both give the one-sided sweep's lists."""
     from swann_amd import _lib
@@ -1119,7 +1119,7 @@ def test_symmetric_sweep_returns_before_the_gpu_is_done(d, dtype):
     assert (gi != wi).float().mean() < 1e-3
 
 
-@pytest.mark.parametrize("n", [9000, 49200])
+@pytest.mark.parametrize("n", [9000, 262000])
 @pytest.mark.parametrize("d,dtype", [(64, "f16"), (100, "f32")])
 def test_sweep_of_any_size_under_graph_capture(n, d, dtype):
     """Sizes whose rows may be ordered (recorded one-sided) and widths swept as three
