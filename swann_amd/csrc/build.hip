@@ -1072,13 +1072,14 @@ int sweep_cap(int C) {
 // at ragged widths with few products, C = 128, in ms, SIMT against MFMA: fp16 150 x
 // 33 0.047 to 0.055, 300 x 33 0.078 to 0.100, 480 x 33 0.107 to 0.100, 300 x 65 0.102
 // to 0.101; fp32 (whose MFMA lists are re-ranked) 150 x 201 0.115 to 0.131, 300 x 150
-// 0.157 to 0.17, 480 x 100 0.178 to 0.18, 576 x 100 0.223 to 0.205.
+// 0.157 to 0.17, 300 x 185 0.183 to 0.18 (C = 256 0.182 to 0.195), 480 x 100 0.178 to
+// 0.18, 576 x 100 0.223 to 0.205.
 constexpr int kRerankMax = 16384;
 constexpr int kSplitMin = 64;
 bool use_mfma(int64_t n, int dim, int x_dtype, int C) {
     const bool f32 = x_dtype == SWANN_DTYPE_F32;
     if (dim % 8 == 0) return true;
-    if (n <= sweep_cap(C) - kCT && n * dim <= (f32 ? 48000 : 12000)) return false;
+    if (n <= sweep_cap(C) - kCT && n * dim <= (f32 ? 56000 : 12000)) return false;
     return !f32 || (dim >= kSplitMin && dim <= kRerankMax);
 }
 

@@ -1170,7 +1170,7 @@ def test_only_overflowed_panels_are_swept_again(opt, d, fcap):
 
 @pytest.mark.parametrize("dtype", ["f16", "f32"])
 @pytest.mark.parametrize("n,d,C", [(2, 5, 1), (2, 64, 2), (65, 7, 65), (240, 50, 20), (241, 50, 20),
-                                   (468, 25, 20), (469, 25, 20), (480, 100, 128), (481, 100, 128),
+                                   (468, 25, 20), (469, 25, 20), (560, 100, 128), (561, 100, 128),
                                    (576, 20, 128), (577, 20, 128), (704, 64, 224), (896, 72, 128),
                                    (897, 72, 128), (832, 64, 32), (833, 64, 32), (788, 33, 20),
                                    (789, 33, 20), (992, 16, 224), (1025, 16, 224),
