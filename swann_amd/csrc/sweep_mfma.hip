@@ -2421,9 +2421,8 @@ inline bool capturing(hipStream_t st) {
 // about 0.618 n and prime to n, so that every panel is an even sample of the corpus.
 // A launch's second lists hold what beats the thresholds the last merge left, and
 // those are only as good as the panels seen: in an order the distances follow (rows
-// sorted by norm, along a line, by cluster) the panels seen say little of the next
-// ones, nearly all of which then beat them, and every list overflows and is swept
-// again.  C = 128, own order and spread (one-sided), ms: rows by rising norm, l2,
+// sorted by norm or along a line) the panels seen say little of the next ones, nearly
+// all of which then beat them, and every list overflows and is swept again.  C = 128, own order and spread (one-sided), ms: rows by rising norm, l2,
 // 8,000 x 768 fp16 4.93 and 0.74 (0.98), 60,000 134.6 and 6.5 (10.7), 60,000 x 100
 // fp32 97.1 and 7.3 (27.6); along a line, ip, 20,000 x 64 fp16 21.3 and 1.4 (5.4).
 // Rows in no order pay for the copy: 60,000 x 768 fp16 7.03 to 7.10, 100,000 x 1,536
